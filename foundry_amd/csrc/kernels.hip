@@ -12,9 +12,10 @@
 //   k_node_b  one workgroup per graph: clean nodes completed from the
 //             template's results, chunk CRCs joined into the node-type and
 //             kernel-entry digests, word offsets by block scans, the
-//             diff-tile -> first-node table, ragged-word sources, slot
+//             diff-tile -> first-node table, slot
 //             descriptors; beside them, one wave per 4 KB slice of every key
 //             and dependency table: their CRC-64/XZ digests.
+//   k_aux     ragged nodes only: where each of their words lies in the file.
 //   k_diff_t  the template graphs' words, relocated through the line-indexed
 //             interval search into R and the live image (1024-word units);
 //             the key-digest collision report.
@@ -645,27 +646,6 @@ __device__ void block_excl_scan2(const uint32_t v[2], uint32_t (*s_tmp)[16], uin
   lds_barrier();
 }
 
-template <class GR>
-__device__ void write_aux(const uint8_t* img, const GR& G, const uint8_t* e, const Side& s, uint64_t* aux,
-                          uint32_t gword) {
-  uint32_t idx = 0;
-  auto put = [&](uint64_t byte, uint32_t size) {
-    for (uint32_t m = 0; m < size; m += 8, ++idx) {
-      if ((uint64_t)gword + idx >= G.word_cap) return;
-      const uint32_t width = min(8u, size - m);
-      aux[G.word_base + gword + idx] = ((byte + m) << 4) | width;
-    }
-  };
-  if (s.extra) {
-    put(s.src, s.arg_size);
-  } else {
-    for (uint32_t j = 0; j < s.num_params; ++j)
-      put(G.sec_off[FDY_SEC_PARAM_DATA] + ld_u32(s.pidx + 8ull * j), ld_u32(s.pidx + 8ull * j + 4));
-  }
-  (void)img;
-  (void)e;
-}
-
 // The node pass runs in two parts.
 //
 // Part A, k_node_a: one workgroup of kNodeChunk threads per chunk of a
@@ -687,8 +667,8 @@ __device__ void write_aux(const uint8_t* img, const GR& G, const uint8_t* e, con
 //     records.
 // Part B, k_node_b: one workgroup per graph: clean nodes completed from the
 // template's results, the chunk CRCs shifted to their place, word offsets
-// by block scans, the tile -> first-node table, ragged-word sources,
-// flatness, status, digests and the slot descriptors of the diff pass.
+// by block scans, the tile -> first-node table, flatness,
+// status, digests and the slot descriptors of the diff pass.
 
 constexpr uint32_t kEntryWords = 168 / 8;  // 8-byte words of a node entry
 constexpr uint32_t kStrStage = 2048;       // string sections up to this size are staged in LDS
@@ -1288,7 +1268,6 @@ __global__ __launch_bounds__(kNodeThreads, 6) void k_node_b(RestoreArgs a) {
   const uint32_t g = blockIdx.x;
   const uint32_t t = *readonly(a.template_of + g);  // written by the grouping pass
   const bool is_t = t == g;
-  const DevGraph& Gg = a.graphs[g];
   // The record fields this pass uses, read through the constant address
   // space: nothing writes the records during the restore, so these are
   // scalar loads, which neither wait for the vector loads in flight nor
@@ -1304,7 +1283,6 @@ __global__ __launch_bounds__(kNodeThreads, 6) void k_node_b(RestoreArgs a) {
   const uint32_t g_word_cap = cg->word_cap, t_word_cap = ct->word_cap;
   const uint32_t g_tile_base = cg->tile_base, g_tile_cap = cg->tile_cap;
   const uint64_t g_word_base = cg->word_base, t_word_base = ct->word_base;
-  const uint8_t* img = a.img;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // A block of kNodeThreads nodes' inputs: the node's first-pass results
   // and, for a member, its template node's (loaded for every node, not only
@@ -1452,15 +1430,9 @@ __global__ __launch_bounds__(kNodeThreads, 6) void k_node_b(RestoreArgs a) {
         uint64_t k = ((uint64_t)gword + kTileWords - 1) / kTileWords;
         const uint64_t k_last = ((uint64_t)gword + words_g - 1) / kTileWords;
         for (; k <= k_last && k < g_tile_cap; ++k) a.tile_node[g_tile_base + k] = n;
-        if (flags & FDY_NODE_RAGGED) {
-          const uint8_t* eg = img + Gg.sec_off[FDY_SEC_NODES] + 168ull * n;
-          Side sd_{}, none_{};
-          bool same_;
-          side_header(img, Gg, RawEntry{eg}, sd_);
-          scan_params(img, Gg, sd_, true, Gg, none_, false, &same_);
-          if (a.aux) write_aux(img, Gg, eg, sd_, a.aux, gword);
-          else atomicOr(a.restore_flags, kFlagNeedAux);  // the host restores again with ragged-word sources
-        }
+        // k_aux records where a ragged node's words lie; without the array for
+        // them the host restores again with it.
+        if ((flags & FDY_NODE_RAGGED) && !a.aux) atomicOr(a.restore_flags, kFlagNeedAux);
       }
     }
     gcarry += tot_g;
@@ -1520,6 +1492,78 @@ __global__ __launch_bounds__(kNodeThreads, 6) void k_node_b(RestoreArgs a) {
     a.slot_desc[g_tile_base + k] = sd;
     a.slot_spill[g_tile_base + k] = 0;
     if (is_t && k < first_unused) a.tslot_desc[s_tbase + k] = sd;
+  }
+}
+
+// Ragged-word sources (archives with ragged nodes only): word w of a ragged
+// node takes `width` bytes from byte `byte` of the image, recorded as
+// byte << 4 | width at the word's place, for the diff passes.
+//   Sixteen lanes per node, one node per lane group: they load a batch of
+// sixteen param entries together, place them by a prefix sum, and then take
+// the batch's words in turn, each finding its param by a binary search over
+// the lanes' sums, so that a node's entries are two dependent loads and its
+// words are stored as whole lines.  Bound by latency (entry, param entries,
+// stores) and by the 8 bytes stored per word.  As part of the second node
+// pass (one thread per node walking its params and words in turn, on as many
+// workgroups as there are graphs) this took 258 us of that pass's 270 on 48
+// graphs x 1237 nodes (3.3 M words); it takes 13 us here.
+constexpr uint32_t kAuxLanes = 16;
+constexpr uint32_t kAuxThreads = 256;
+constexpr uint32_t kAuxNodes = kAuxThreads / kAuxLanes;  // nodes per workgroup and step
+constexpr uint32_t kAuxUnits = kNodeChunk / kAuxNodes;   // steps per node chunk
+static_assert(kNodeChunk % kAuxNodes == 0, "whole steps per chunk");
+
+__global__ __launch_bounds__(kAuxThreads) void k_aux(RestoreArgs a) {
+  const uint32_t l = threadIdx.x % kAuxLanes;
+  const uint32_t units = a.num_chunks * kAuxUnits;  // below 2^29: an archive holds fewer than 2^32 nodes
+  for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
+    const uint32_t chunk = u / kAuxUnits;
+    const ConstGraph& G = *readonly(a.graphs + *readonly(reinterpret_cast<const uint32_t*>(a.chunk_gt + chunk)));
+    const uint32_t N = G.num_nodes;
+    const uint32_t pad = (kNodeChunk - N % kNodeChunk) % kNodeChunk;  // a graph's chunks end at its last node
+    const int64_t n = (int64_t)(chunk - G.chunk_base) * kNodeChunk - pad + (u % kAuxUnits) * kAuxNodes +
+                      threadIdx.x / kAuxLanes;
+    if (n < 0 || n >= (int64_t)N) continue;  // the same for a node's sixteen lanes
+    const uint4 d = *reinterpret_cast<const uint4*>(a.node_desc + G.node_base + n);  // gword, nwords, tword, flags
+    if (!(d.w & FDY_NODE_RAGGED) || d.y == 0 || d.x >= G.word_cap) continue;
+    const uint32_t room = G.word_cap - d.x;  // words of this node inside the image
+    uint64_t* out = a.aux + G.word_base + d.x;
+    Side s;
+    side_header(a.img, G, RawEntry{a.img + G.sec_off[FDY_SEC_NODES] + 168ull * (uint64_t)n}, s);
+    if (s.extra) {
+      const uint32_t words = min(s.words, room);
+      for (uint32_t w = l; w < words; w += kAuxLanes)
+        out[w] = ((s.src + 8ull * w) << 4) | min(8u, s.arg_size - 8 * w);
+      continue;
+    }
+    const uint64_t base = G.sec_off[FDY_SEC_PARAM_DATA];
+    uint32_t at = 0;  // words before this batch (sums saturate: past `room` nothing is stored)
+    for (uint32_t jb = 0; jb < s.num_params && at < room; jb += kAuxLanes) {
+      const uint32_t j = jb + l;
+      const uint64_t e = ld_u64_any(s.pidx + 8ull * (j < s.num_params ? j : 0));
+      const uint32_t off = (uint32_t)e, size = j < s.num_params ? (uint32_t)(e >> 32) : 0;
+      const uint32_t own = size / 8 + (size % 8 != 0);
+      uint32_t end = own;  // words of the batch up to and with this lane's param
+#pragma unroll
+      for (uint32_t k = 1; k < kAuxLanes; k <<= 1) {
+        const uint32_t y = __shfl_up(end, k, kAuxLanes);
+        if (l >= k) end = __builtin_elementwise_add_sat(end, y);
+      }
+      const uint32_t total = __shfl(end, kAuxLanes - 1, kAuxLanes);
+      const uint32_t words = min(total, room - at);
+      // Every lane takes part in each step's exchanges.
+      for (uint32_t w0 = 0; w0 < words; w0 += kAuxLanes) {
+        const uint32_t w = w0 + l;
+        uint32_t q = 0;  // the param holding word w: the first whose end lies past it
+#pragma unroll
+        for (uint32_t k = kAuxLanes / 2; k; k >>= 1)
+          if (__shfl(end, q + k - 1, kAuxLanes) <= w) q += k;
+        const uint32_t m = 8 * (w - (__shfl(end, q, kAuxLanes) - __shfl(own, q, kAuxLanes)));
+        const uint32_t po = __shfl(off, q, kAuxLanes), ps = __shfl(size, q, kAuxLanes);
+        if (w < words) out[at + w] = ((base + po + m) << 4) | min(8u, ps - m);
+      }
+      at = __builtin_elementwise_add_sat(at, total);
+    }
   }
 }
 
@@ -2673,6 +2717,12 @@ hipError_t launch_node(const RestoreArgs& a, hipStream_t s) {
   }
   const uint32_t unit_blocks = (a.num_units + kNodeThreads / 64 - 1) / (kNodeThreads / 64);
   hipLaunchKernelGGL(k_node_b, dim3(a.num_graphs + unit_blocks), dim3(kNodeThreads), 0, s, a);
+  if (a.aux && a.num_chunks) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const uint32_t grid = std::min(a.num_chunks * kAuxUnits, 1u << 16);
+    hipLaunchKernelGGL(k_aux, dim3(grid), dim3(kAuxThreads), 0, s, a);
+  }
   return hipGetLastError();
 }
 
