@@ -61,11 +61,12 @@ struct DevBuf {
 
 int dev_alloc(DevBuf& b, size_t bytes, const char* what);
 
-// The interval search structure: an index of 64-byte lines, one to two
-// root lines per interval, each answering the searches inside it or naming
-// the lines that do (see RelocLine).
+// The interval search structure: the two-level index of a table (RelocRoot,
+// RelocLine) in one allocation, root entries first, or its index of root
+// lines.  `table`: lo, hi and new_lo on the device, kept where the index of
+// root lines may yet be asked for.
 struct RelocPlan {
-  DevBuf line;
+  DevBuf index, table;
   RelocDev dev{};
 };
 

@@ -120,28 +120,38 @@ struct MirrorArgs {
 constexpr uint32_t kMirrorNodes = 64;  // nodes per block
 hipError_t launch_mirror(const MirrorArgs& a, hipStream_t s);
 
+// Relocates packed words through the table's two-level index, or (r.root
+// null and more than one interval) through its root lines.
 hipError_t launch_reloc_words(const RelocDev& r, const uint64_t* in, uint64_t* out, uint64_t n, hipStream_t s);
 
-// The interval index built on the device (the builder of reloc_index.h, one
-// thread per root line): launch_index_count writes each workgroup's first
-// line below its roots into block_sum (one per kIndexThreads root lines) and
-// the index's line count into *total; launch_index_place then writes the
-// lines (line holds *total of them).
+// A table's index built on the device (the builders of reloc_index.h).  The
+// count launches write each workgroup's first line into block_sum and the
+// line count into *total; the place launches then write the entries and
+// lines (line holds *total of them).  launch_roots_*: the two-level index,
+// kRootBlock root entries per workgroup.  launch_index_*: the index of root
+// lines, one thread per root line, kIndexThreads per workgroup.
 constexpr uint32_t kIndexThreads = 64;  // one wave: 24 KB of LDS for the subtree counts
+constexpr uint32_t kRootBlock = 256;
 struct IndexArgs {
   const uint64_t* lo;   // the table, on the device
   const uint64_t* hi;
   const uint64_t* nlo;
   uint64_t n;           // intervals (> 0)
-  uint64_t nb;          // root lines
-  uint32_t shift;       // root line width: 2^shift bytes
+  uint64_t nb;          // root lines, or root entries
+  uint32_t shift;       // their width: 2^shift bytes
+  uint32_t fence_shift; // two-level index: the fences' unit
+  uint32_t exact;       // two-level index: every start is on that unit
   uint32_t pad_;
-  uint64_t* block_sum;  // ceil(nb / kIndexThreads) entries
+  uint32_t* ends;       // two-level index: per root entry, the intervals starting before its range's end
+  uint64_t* block_sum;  // one per workgroup of the count launch
   uint64_t* total;
+  RelocRoot* root;      // two-level index
   RelocLine* line;
 };
 hipError_t launch_index_count(const IndexArgs& a, hipStream_t s);
 hipError_t launch_index_place(const IndexArgs& a, hipStream_t s);
+hipError_t launch_roots_count(const IndexArgs& a, hipStream_t s);
+hipError_t launch_roots_place(const IndexArgs& a, hipStream_t s);
 
 // A memset node of a restored graph, run as a kernel node: `height` rows of
 // `row_bytes` bytes, `pitch` bytes apart, each byte k of a row taking byte

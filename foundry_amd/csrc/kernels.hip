@@ -16,7 +16,7 @@
 //             descriptors; beside them, one wave per 4 KB slice of every key
 //             and dependency table: their CRC-64/XZ digests.
 //   k_aux     ragged nodes only: where each of their words lies in the file.
-//   k_diff_t  the template graphs' words, relocated through the line-indexed
+//   k_diff_t  the template graphs' words, relocated through the indexed
 //             interval search into R and the live image (1024-word units);
 //             the key-digest collision report.
 //   k_diff_m  eight workgroups per 4096-word tile of every other graph: coalesced
@@ -34,9 +34,11 @@
 //   k_mirror  dirty nodes' live words -> a group graph's host mirror.
 //   k_fill    memset node of a restored graph, as a kernel node.
 //   k_reloc   streaming relocation of packed words.
+//   k_roots_count, k_index_scan, k_roots_place
+//             the two-level interval index of a relocation table, a thread
+//             per root entry and per line (the builder of reloc_index.h).
 //   k_index_count, k_index_scan, k_index_place
-//             the interval index of a relocation table, one thread per root
-//             line (the builder of reloc_index.h).
+//             its index of root lines, a thread per root line.
 #include <type_traits>
 
 #include "kernels.h"
@@ -61,6 +63,11 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* readonly(c
 constexpr uint32_t kNodeThreads = 512;
 constexpr uint32_t kRelocThreads = 256;
 constexpr uint32_t kRelocPairs = 4;  // 16-byte word pairs per thread per iteration
+// Calls of fewer words than fill the GPU twice over take one pair per thread,
+// so that a small call (a graph's params) spreads over four times the
+// workgroups and a wave searches for 32 words at a time instead of 128.
+constexpr uint64_t kRelocFewWords = 2ull * 256 * kRelocThreads * 2 * kRelocPairs;
+constexpr uint32_t kRelocBlocks = 256 * 32;
 
 __device__ inline uint64_t shfl_down64(uint64_t v, int d) {
   uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
@@ -790,6 +797,7 @@ __device__ __forceinline__ void node_full(const RestoreArgs& a, const GR& Gg, co
 
 // Two consecutive 8-byte words as one 16-byte access at 8-byte alignment
 // (gfx950 serves a 16-byte global access at any 4-byte alignment).
+typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 typedef uint64_t u64x2a8 __attribute__((ext_vector_type(2), aligned(8)));
 
 // Write-once results that no pass of the restore reads back soon (the
@@ -1691,6 +1699,138 @@ __device__ inline uint64_t load_word(const RestoreArgs& a, const GR& G, const No
   return *reinterpret_cast<const uint64_t*>(a.img + src + 8ull * (w - d.gword));
 }
 
+// Orders a wave's own LDS accesses: what it wrote before is what it reads
+// after (the wave runs in program order; this keeps the compiler's).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The lanes below this one in `mask`.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+
+// The interval searches of a wave: the words sw[pos[0 .. cnt)] (LDS; every
+// one inside the table's range, and the table has more than one interval) are
+// relocated in place.  lx: kSearchBatch entries of the wave's LDS.
+//   The root entries are gathered a lane per word; the lanes whose entry
+// answers add its delta, those whose entry has a tree descend it to their
+// leaf.  The leaves are then read four lanes per
+// word, one slot each, so that a load instruction takes 16 whole lines, and
+// the lane whose slot holds the word (its start at or before it, the next
+// lane's past it) adds the slot's delta to the word in LDS.  kLines lines per
+// quad are in flight.
+//   Bound by requests: 4 ps each over the GPU where they hit the L2s, 18 ps
+// where they miss them, whatever their size up to 128 B (250 and 55 G/s
+// measured over 4 MB and 200 MB).  So the index is small (about 25 bytes per
+// interval up to 64,000 of them) and one more, cached, read deep.  20.5 M
+// words with 25% pointers by 40,000 intervals: 97 us, where 16 root lines of
+// 64 B per interval (41 MB) read by one lane each took 136 us; eight lanes per
+// 128-byte line were slower than four per 64 bytes (an L2 hit delivers 10.5
+// TB/s, so 128 B cost 12 ps).
+constexpr uint32_t kSearchBatch = 128;
+
+template <int kPerm>
+__device__ __forceinline__ uint32_t quad_perm(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kPerm, 0xF, 0xF, true);
+}
+__device__ __forceinline__ uint32_t quad_first(uint32_t v) { return quad_perm<0x00>(v); }
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) {
+  v += quad_perm<0xB1>(v);         // lanes 1, 0, 3, 2
+  return v + quad_perm<0x4E>(v);   // lanes 2, 3, 0, 1
+}
+__device__ __forceinline__ uint32_t quad_max(uint32_t v) {
+  v = max(v, quad_perm<0xB1>(v));
+  return max(v, quad_perm<0x4E>(v));
+}
+
+template <uint32_t kLines, bool kRooted = true>
+__device__ __forceinline__ void wave_search(const RelocDev& R, uint64_t* sw, const uint16_t* pos, uint2* lx,
+                                            uint32_t cnt) {
+  const uint32_t lane = threadIdx.x & 63, quad = lane >> 2, part = lane & 3;
+  wave_fence();
+#pragma unroll 1
+  for (uint32_t b = 0; b < cnt; b += kSearchBatch) {
+    constexpr uint32_t K = kSearchBatch / 64;
+    uint32_t x[K];
+    uint4 rt[K];
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+      const uint64_t rel = sw[pos[min(b + 64 * k + lane, cnt - 1)]] - R.lo_min;
+      const uint64_t r = rel >> R.shift;
+      x[k] = (uint32_t)(rel - (r << R.shift));
+      if constexpr (kRooted) rt[k] = *reinterpret_cast<const uint4*>(R.root + r);
+      else rt[k].x = (uint32_t)r;  // its root line
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+      uint32_t line = rt[k].x;
+      if constexpr (kRooted) {
+        const uint32_t x0 = x[k];
+        line = root_child(rt[k], R.fence_shift, &x[k]);
+        if ((rt[k].x & kRootDirect) && b + 64 * k + lane < cnt && slot_holds(R, x0, rt[k].y))
+          sw[pos[b + 64 * k + lane]] += (uint64_t)rt[k].z | ((uint64_t)rt[k].w << 32);
+        if (rt[k].x & kRootTree) line = tree_leaf(R, line, &x[k]);
+      }
+      lx[64 * k + lane] = make_uint2(line, x[k]);
+    }
+    wave_fence();
+    const uint32_t end = min(cnt - b, kSearchBatch);
+#pragma unroll 1
+    for (uint32_t i0 = 0; i0 < end; i0 += 16 * kLines) {
+      uint4 q[kLines];
+      uint32_t x4[kLines];
+#pragma unroll
+      for (uint32_t u = 0; u < kLines; ++u) {
+        const uint2 e = lx[i0 + 16 * u + quad];
+        x4[u] = e.y;
+        q[u] = reinterpret_cast<const uint4*>(R.line + e.x)[part];
+      }
+      // Every lane needs its whole slot: left to itself the compiler loads
+      // the delta again, behind the branch that adds it.
+#pragma unroll
+      for (uint32_t u = 0; u < kLines; ++u)
+        asm volatile("" : "+v"(q[u].x), "+v"(q[u].y), "+v"(q[u].z), "+v"(q[u].w));
+      if constexpr (!kRooted) {
+        // A root line that is a fence line: to the child after the last fence
+        // at or before x, all the quads' lines of a level together.
+        for (;;) {
+          uint32_t kind = 0;
+#pragma unroll
+          for (uint32_t u = 0; u < kLines; ++u) kind |= quad_first(q[u].x);
+          if (!__ballot(kind & kLineFence)) break;
+#pragma unroll
+          for (uint32_t u = 0; u < kLines; ++u) {
+            if (!(quad_first(q[u].x) & kLineFence)) continue;  // the quad's four lanes alike
+            const uint4 L = q[u];
+            // Part 0's first two words are the kind and the first child.
+            const bool l0 = part && L.x <= x4[u], l1 = part && L.y <= x4[u], l2 = L.z <= x4[u], l3 = L.w <= x4[u];
+            const uint32_t c = quad_sum((uint32_t)l0 + l1 + l2 + l3);
+            x4[u] -= quad_max(l3 ? L.w : l2 ? L.z : l1 ? L.y : l0 ? L.x : 0u);
+            q[u] = reinterpret_cast<const uint4*>(R.line + quad_first(L.y) + c)[part];
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kLines; ++u)
+            asm volatile("" : "+v"(q[u].x), "+v"(q[u].y), "+v"(q[u].z), "+v"(q[u].w));
+        }
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kLines; ++u) {
+        const uint32_t i = i0 + 16 * u + quad, x = x4[u];
+        // The next lane's start (lane 3 of the quad reads itself).
+        const uint32_t nx = quad_perm<0xF9>(q[u].x);
+        const uint32_t past = part == 3 ? kLineNone : nx;
+        if (i < end && q[u].x <= x && x < past && slot_holds(R, x, q[u].y))  // a leaf's slot 0 starts at 0
+          atomicAdd(reinterpret_cast<unsigned long long*>(sw + pos[b + i]),
+                    (unsigned long long)q[u].z | ((unsigned long long)q[u].w << 32));
+      }
+    }
+    wave_fence();
+  }
+}
+
 // Template graphs: relocate their words into R and the live image.  The
 // template slots listed by the node pass are cut into units of kTUnit words
 // (kTWords per thread, so one search batch), spread over the grid.  Four
@@ -1699,6 +1839,7 @@ __device__ inline uint64_t load_word(const RestoreArgs& a, const GR& G, const No
 // turn) measured 108 -> 97 us on the MoE-style archive, while four keep the
 // decode-style pass at 10.9 us (13.0 us with eight).
 constexpr uint32_t kTThreads = 256;
+constexpr uint32_t kTLines = 8;  // lines in flight per quad
 constexpr uint64_t kTWideSlotsPerGraph = 64;  // 64 slots of 4096 words: 256K words per graph
 template <uint32_t kTWords>
 constexpr uint32_t t_units_per_tile() {
@@ -1706,16 +1847,16 @@ constexpr uint32_t t_units_per_tile() {
   return kTileWords / (kTThreads * kTWords);
 }
 
-constexpr uint32_t kTSearch = 2;  // searches per lane in one lockstep batch
-
 template <uint32_t kTWords>
 __global__ __launch_bounds__(kTThreads) void k_diff_t(RestoreArgs a) {
   constexpr uint32_t kTUnit = kTThreads * kTWords;
   constexpr uint32_t kTUnitsPerTile = t_units_per_tile<kTWords>();
   __shared__ NodeDesc s_nd[kDiffWindow];
-  __shared__ uint64_t s_q[kTThreads / 64][64 * kTWords];  // per wave: the words it searches
+  // Per wave: its words, the places of those it searches, their lines.
+  __shared__ uint64_t s_w[kTThreads / 64][64 * kTWords];
+  __shared__ uint16_t s_pos[kTThreads / 64][64 * kTWords];
+  __shared__ uint2 s_lx[kTThreads / 64][kSearchBatch];
   const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const uint64_t lt = (1ull << lane) - 1;
   const RelocDev& R = a.reloc;
   const uint32_t units = *readonly(a.tslot_count) * kTUnitsPerTile;
   // The next unit's slot descriptor is loaded while this unit is worked on
@@ -1730,7 +1871,7 @@ __global__ __launch_bounds__(kTThreads) void k_diff_t(RestoreArgs a) {
     const uint64_t ubeg = (uint64_t)sd.wbeg + (u % kTUnitsPerTile) * kTUnit;
     const uint64_t uend = min((uint64_t)sd.wend, ubeg + kTUnit);
     if (ubeg >= uend) continue;  // uniform over the block
-    uint64_t v[kTWords], r[kTWords];
+    uint64_t v[kTWords];
     uint32_t m = 0;
     if (sd.flags & kSlotFlat) {
       const uint8_t* pg = a.img + sd.kg;
@@ -1768,54 +1909,33 @@ __global__ __launch_bounds__(kTThreads) void k_diff_t(RestoreArgs a) {
     }
     // The whole words inside the table's range need an interval search:
     // about a quarter of them on the presets (the pointers).  Each wave
-    // compacts its words to search in LDS, searches them kTSearch per lane
-    // in lockstep, and every lane reads its results back, so no lane holds
-    // line registers for words that need no search.
-    uint32_t need = 0;
-    if (R.n != 0) {
+    // lists them in LDS and searches them there.
+    if (R.n > 1) {
+      uint64_t* sw = s_w[tid >> 6];
+      uint16_t* pos = s_pos[tid >> 6];
+      uint32_t cnt = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < kTWords; ++q) {
+        const bool need = ((m >> q) & 1) && reloc_in_range(R, v[q]);
+        const uint64_t mk = __ballot(need);
+        sw[64 * q + lane] = v[q];
+        if (need) pos[cnt + lanes_below(mk)] = (uint16_t)(64 * q + lane);
+        cnt += (uint32_t)__popcll(mk);
+      }
+      wave_search<kTLines>(R, sw, pos, s_lx[tid >> 6], cnt);
+#pragma unroll
+      for (uint32_t q = 0; q < kTWords; ++q) v[q] = sw[64 * q + lane];
+      wave_fence();  // the next unit's words follow every lane's reads
+    } else {
 #pragma unroll
       for (uint32_t q = 0; q < kTWords; ++q)
-        if (((m >> q) & 1) && v[q] >= R.lo_min && (R.policy ? v[q] <= R.hi_max : v[q] < R.hi_max)) need |= 1u << q;
+        if ((m >> q) & 1) v[q] = reloc_word(R, v[q]);
     }
-    uint64_t* sq = s_q[tid >> 6];
-    uint32_t rank[kTWords], cnt = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < kTWords; ++q) {
-      const uint64_t mk = __ballot((need >> q) & 1);
-      rank[q] = cnt + (uint32_t)__popcll(mk & lt);
-      if ((need >> q) & 1) sq[rank[q]] = v[q];
-      cnt += (uint32_t)__popcll(mk);
-    }
-    // The wave's own LDS words: its writes precede its reads in program order.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (uint32_t b = 0; b < cnt; b += 64 * kTSearch) {
-      uint64_t x[kTSearch], y[kTSearch];
-      uint32_t mm = 0;
-#pragma unroll
-      for (uint32_t k = 0; k < kTSearch; ++k) {
-        const uint32_t i = b + 64 * k + lane;
-        x[k] = i < cnt ? sq[i] : 0;
-        mm |= (i < cnt ? 1u : 0u) << k;
-      }
-      reloc_batch<kTSearch>(R, x, y, mm);
-#pragma unroll
-      for (uint32_t k = 0; k < kTSearch; ++k) {
-        const uint32_t i = b + 64 * k + lane;
-        if (i < cnt) sq[i] = y[k];
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (uint32_t q = 0; q < kTWords; ++q) r[q] = ((need >> q) & 1) ? sq[rank[q]] : v[q];
     uint64_t* img_out = a.image + sd.word_base;
 #pragma unroll
     for (uint32_t q = 0; q < kTWords; ++q) {
       const uint64_t w = ubeg + q * kTThreads + tid;
-      if (w < uend) img_out[w] = r[q];
+      if (w < uend) img_out[w] = v[q];
     }
   }
   // The collision report, one graph per workgroup in turn, from the last
@@ -1852,7 +1972,6 @@ __global__ __launch_bounds__(kTThreads) void k_diff_t(RestoreArgs a) {
 constexpr uint32_t kMSplit = 8;
 constexpr uint32_t kMThreads = kSubsPerSlot * 64 / kMSplit;
 static_assert(kSubsPerSlot % kMSplit == 0, "whole sub-ranges per workgroup");
-constexpr uint32_t kSlots = 2;  // searches per batch in the overflowed-template path
 
 // Six waves per SIMD: the node window in LDS (12 KB per workgroup) allows
 // no more.
@@ -1970,14 +2089,14 @@ __global__ __launch_bounds__(kMThreads, 6) void k_diff_m(RestoreArgs a) {
     for (uint32_t j = 0; j < J; ++j) fr[j] = ft[j];  // relocation off: R equals the raw image
   } else if (t_status & kGraphOverflow) {
     // The template overflowed its capacity: relocate its compared words here.
+#pragma unroll 1
+    for (uint32_t j = 0; j < J; ++j) {
+      uint64_t o = 0;  // ft[j], without indexing the registers
 #pragma unroll
-    for (uint32_t jb = 0; jb < J; jb += kSlots) {
-      uint64_t tin[kSlots], tout[kSlots];
+      for (uint32_t k = 0; k < J; ++k) o = k == j ? ft[k] : o;
+      if (((cmp & full) >> j) & 1) o = reloc_word(R, o);
 #pragma unroll
-      for (uint32_t k = 0; k < kSlots; ++k) tin[k] = ft[jb + k];
-      reloc_batch<kSlots>(R, tin, tout, ((cmp & full) >> jb) & ((1u << kSlots) - 1));
-#pragma unroll
-      for (uint32_t k = 0; k < kSlots; ++k) fr[jb + k] = tout[k];
+      for (uint32_t k = 0; k < J; ++k) fr[k] = k == j ? o : fr[k];
     }
   }
 
@@ -2101,6 +2220,7 @@ __global__ __launch_bounds__(kMThreads, 6) void k_diff_m(RestoreArgs a) {
 // makes no record and leaves a gap at the end of its slot's range: the slot
 // raises the archive's gap flag, and k_repack closes the gaps before any
 // result is read.  The slot's record count goes to slot_rec.
+constexpr uint32_t kSLines = 4;  // lines in flight per quad
 constexpr uint32_t kSThreads = 256;  // four slots per workgroup
 constexpr uint32_t kSBatch = 128;  // two per lane: three or four per lane measured 1.8 and 4.4 times slower
 
@@ -2141,10 +2261,16 @@ __global__ __launch_bounds__(kSThreads, 6) void k_diff_s(RestoreArgs a) {
   // Per wave: {first graph word, first template word} of its window's nodes.
   __shared__ uint2 s_win[kSThreads / 64][kDiffWindow];
   __shared__ uint32_t s_off[kSThreads / 64][kSubsPerSlot];
+  // Per wave: a batch's words, the places of those it searches, their lines.
+  __shared__ uint64_t s_w[kSThreads / 64][kSBatch];
+  __shared__ uint16_t s_pos[kSThreads / 64][kSBatch];
+  __shared__ uint2 s_lx[kSThreads / 64][kSearchBatch];
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t slot = blockIdx.x * (kSThreads / 64) + (threadIdx.x >> 6);
   if (slot >= a.num_slots) return;  // per wave: this kernel has no barrier
   uint2* const s_gt = s_win[threadIdx.x >> 6];
+  uint64_t* const sw = s_w[threadIdx.x >> 6];
+  uint16_t* const pos = s_pos[threadIdx.x >> 6];
   uint32_t* counts = a.sub_count + (uint64_t)slot * kSubsPerSlot;
   // What depends on the slot alone is loaded first.
   const uint32_t cnt = lane < kSubsPerSlot ? counts[lane] : 0;
@@ -2264,7 +2390,24 @@ __global__ __launch_bounds__(kSThreads, 6) void k_diff_s(RestoreArgs a) {
       fl[kk] = in ? cur[kk].flags : 0;
       if (fl[kk] & kCandReloc) m |= 1u << kk;
     }
-    reloc_batch<K>(a.reloc, raw, res, m);
+    if (a.reloc.n > 1) {  // uniform over the archive
+      uint32_t cnt = 0;
+#pragma unroll
+      for (uint32_t kk = 0; kk < K; ++kk) {
+        const bool need = ((m >> kk) & 1) && reloc_in_range(a.reloc, raw[kk]);
+        const uint64_t mk = __ballot(need);
+        sw[64 * kk + lane] = raw[kk];
+        if (need) pos[cnt + lanes_below(mk)] = (uint16_t)(64 * kk + lane);
+        cnt += (uint32_t)__popcll(mk);
+      }
+      wave_search<kSLines>(a.reloc, sw, pos, s_lx[threadIdx.x >> 6], cnt);
+#pragma unroll
+      for (uint32_t kk = 0; kk < K; ++kk) res[kk] = sw[64 * kk + lane];
+      wave_fence();  // the next batch's words follow every lane's reads
+    } else {
+#pragma unroll
+      for (uint32_t kk = 0; kk < K; ++kk) res[kk] = (m >> kk) & 1 ? reloc_word(a.reloc, raw[kk]) : raw[kk];
+    }
     // The member pass stored each candidate's raw word; only the words the
     // relocation moved are stored again (a scattered 8-byte store costs a
     // partly written line).
@@ -2525,11 +2668,12 @@ __global__ __launch_bounds__(kIndexThreads) void k_index_count(IndexArgs a) {
   if (threadIdx.x == 0) a.block_sum[blockIdx.x] = tot;
 }
 
-// Pass 2, one workgroup of kIndexScanThreads: each root workgroup's first
-// line below its roots (after the nb root lines), and the index's line
-// count.  Each thread sums, then rewrites, a contiguous run of the counts.
+// Pass 2, one workgroup of kIndexScanThreads: each workgroup's first line
+// (from `first` on: the lines below the roots follow the nb root lines), and
+// the index's line count.  Each thread sums, then rewrites, a contiguous run
+// of the counts.
 constexpr uint32_t kIndexScanThreads = 1024;
-__global__ __launch_bounds__(kIndexScanThreads) void k_index_scan(IndexArgs a, uint64_t nblocks) {
+__global__ __launch_bounds__(kIndexScanThreads) void k_index_scan(IndexArgs a, uint64_t nblocks, uint64_t first) {
   __shared__ uint64_t s_part[kIndexScanThreads / 64];
   const uint64_t per = (nblocks + kIndexScanThreads - 1) / kIndexScanThreads;
   const uint64_t k0 = min(nblocks, (uint64_t)threadIdx.x * per), k1 = min(nblocks, k0 + per);
@@ -2537,13 +2681,13 @@ __global__ __launch_bounds__(kIndexScanThreads) void k_index_scan(IndexArgs a, u
 #pragma unroll 8
   for (uint64_t k = k0; k < k1; ++k) v += a.block_sum[k];
   uint64_t tot;
-  uint64_t at = a.nb + index_block_scan<kIndexScanThreads / 64>(v, s_part, &tot);
+  uint64_t at = first + index_block_scan<kIndexScanThreads / 64>(v, s_part, &tot);
   for (uint64_t k = k0; k < k1; ++k) {
     const uint64_t x = a.block_sum[k];
     a.block_sum[k] = at;
     at += x;
   }
-  if (threadIdx.x == 0) *a.total = a.nb + tot;
+  if (threadIdx.x == 0) *a.total = first + tot;
 }
 
 // Pass 3, one thread per root line: the root line and the lines below it.
@@ -2556,6 +2700,105 @@ __global__ __launch_bounds__(kIndexThreads) void k_index_place(IndexArgs a) {
   uint64_t tot;
   const uint64_t base = a.block_sum[blockIdx.x] + index_block_scan<kIndexThreads / 64>(sub, s_part, &tot);
   if (b < a.nb) place_root(a.line, b, s0, i, j, a.lo, a.hi, a.nlo, base);
+}
+
+// The two-level index, one workgroup per kRootBlock root entries.
+//   The count pass finds the intervals starting in the workgroup's range (a
+// 64-way search by one wave for either end: four rounds of loads for 2M
+// intervals, where a binary search per root took 21), reads their starts
+// once, coalesced, and counts them per entry in LDS; a prefix sum gives every
+// entry its interval range, kept for the place pass.  The place pass gives
+// every line a thread: the lines of a workgroup's entries are consecutive,
+// so it stores them as whole runs whatever the entries' sizes are.
+//   Bound by latency at 200,000 intervals (10 us count, 14 us place, 4 us the
+// scan between them, for 5 MB); one thread per root line searching the table
+// and writing its subtree, as the index of root lines is built, takes 180, 250
+// and 59 us there, for 156 MB.
+
+// The first k of [0, n) with lo[k] >= key, by the whole wave.
+__device__ inline uint64_t wave_lower_bound(const uint64_t* lo, uint64_t n, uint64_t key) {
+  const uint32_t lane = threadIdx.x & 63;
+  uint64_t a = 0, c = n;  // in [a, c]
+  while (c - a > 64) {
+    const uint64_t step = (c - a + 63) / 64, p = a + lane * step;
+    const uint32_t below = (uint32_t)__popcll(__ballot(p < c && lo[p < c ? p : c - 1] < key));
+    if (below == 0) return a;
+    c = min(c, a + below * step);
+    a += (below - 1) * step + 1;
+  }
+  const uint64_t p = a + lane;
+  return a + (uint32_t)__popcll(__ballot(p < c && lo[p < c ? p : n - 1] < key));
+}
+
+__global__ __launch_bounds__(kRootBlock) void k_roots_count(IndexArgs a) {
+  __shared__ uint64_t s_part[kRootBlock / 64];
+  __shared__ uint64_t s_end[2];
+  __shared__ uint32_t s_count[kRootBlock];
+  const uint32_t tid = threadIdx.x, wave = tid >> 6;
+  const uint64_t b0 = (uint64_t)blockIdx.x * kRootBlock, b1 = min(a.nb, b0 + kRootBlock), b = b0 + tid;
+  const uint64_t lo0 = a.lo[0];
+  s_count[tid] = 0;
+  if (wave < 2) {
+    const uint64_t k = wave_lower_bound(a.lo, a.n, root_start(lo0, a.shift, wave ? b1 : b0));
+    if ((tid & 63) == 0) s_end[wave] = k;
+  }
+  __syncthreads();
+  const uint64_t first = s_end[0], last = s_end[1];
+  for (uint64_t k = first + tid; k < last; k += kRootBlock) {
+    const uint32_t e = (uint32_t)(((a.lo[k] - lo0) >> a.shift) - b0);
+    // Starts are in order, so a crowded range often gives a wave one entry.
+    const uint32_t e0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)e);
+    const uint64_t here = __ballot(true);
+    if (__ballot(e == e0) == here) {
+      if ((here & ((1ull << (tid & 63)) - 1)) == 0) atomicAdd(&s_count[e], (uint32_t)__popcll(here));
+    } else {
+      atomicAdd(&s_count[e], 1u);
+    }
+  }
+  __syncthreads();
+  const uint32_t own = s_count[tid];
+  uint64_t tot;
+  const uint64_t before = first + index_block_scan<kRootBlock / 64>(own, s_part, &tot);
+  uint64_t below = 0;
+  if (b < a.nb) {
+    a.ends[b] = (uint32_t)(before + own);
+    const uint64_t i = root_first(a.lo, a.n, root_start(lo0, a.shift, b), before);
+    below = root_lines(before + own - i, a.exact);
+  }
+  (void)index_block_scan<kRootBlock / 64>(below, s_part, &tot);
+  if (tid == 0) a.block_sum[blockIdx.x] = tot;
+}
+
+__global__ __launch_bounds__(kRootBlock) void k_roots_place(IndexArgs a) {
+  __shared__ uint64_t s_part[kRootBlock / 64];
+  __shared__ uint64_t s_first[kRootBlock];  // per entry: its first line, within the workgroup's
+  __shared__ uint32_t s_i[kRootBlock], s_j[kRootBlock];
+  const uint32_t tid = threadIdx.x;
+  const uint64_t b0 = (uint64_t)blockIdx.x * kRootBlock, b = b0 + tid;
+  const uint64_t lo0 = a.lo[0], base = a.block_sum[blockIdx.x];
+  uint64_t s0 = 0, i = 0, j = 0, below = 0;
+  if (b < a.nb) {
+    s0 = root_start(lo0, a.shift, b);
+    i = root_first(a.lo, a.n, s0, b ? a.ends[b - 1] : 0u);
+    j = a.ends[b] - 1ull;
+    below = root_lines(j - i + 1, a.exact);
+  }
+  uint64_t tot;
+  const uint64_t first = index_block_scan<kRootBlock / 64>(below, s_part, &tot);
+  s_first[tid] = first;
+  s_i[tid] = (uint32_t)i;
+  s_j[tid] = (uint32_t)j;
+  if (b < a.nb) a.root[b] = root_entry(s0, i, j, a.lo, a.hi, a.nlo, a.fence_shift, a.exact, base + first);
+  if (b == 0) a.line[0] = null_line();
+  __syncthreads();
+  for (uint64_t l = tid; l < tot; l += kRootBlock) {
+    uint32_t e = 0;  // the entry holding line l: the last whose first line is at or before l
+#pragma unroll
+    for (uint32_t h = kRootBlock / 2; h; h >>= 1)
+      if (s_first[e + h] <= l) e += h;
+    place_below(a.line, base + s_first[e], l - s_first[e], root_start(lo0, a.shift, b0 + e), s_i[e], s_j[e], a.lo,
+                a.hi, a.nlo, a.exact);
+  }
 }
 
 // ---- host mirror of a group graph's live image ---------------------------
@@ -2613,92 +2856,80 @@ __global__ __launch_bounds__(kFillThreads) void k_fill(FillArgs a) {
 
 // `in` and `out` may be the same array: each word is read and then written
 // by one thread, so in-place relocation needs no ordering between threads.
-// Standalone relocation of packed words.  Each thread owns kRelocPairs
-// 16-byte pairs per chunk (coalesced across the workgroup).  The words
-// inside the table's range (the pointers: 40% on the relocation-heavy
-// workload) are compacted per wave in LDS and searched kRelocSearch per lane
-// in lockstep, then read back in place, so no lane holds index lines for
-// words that need no search: 90 VGPRs and five waves per SIMD, where
-// searching every word in batches of four took 148 VGPRs and three.
-constexpr uint32_t kRelocSearch = 2;
-static_assert((64 * 2 * kRelocPairs) % (64 * kRelocSearch) == 0, "whole search batches per wave");
+// Standalone relocation of packed words.  Each thread owns kPairs
+// 16-byte pairs per chunk (coalesced across the workgroup; 8-byte aligned
+// arrays too), and loads its next chunk's before it searches for this one's.
+// A wave's words lie in LDS meanwhile, with a list of those inside the
+// table's range (the pointers: 40% on the relocation-heavy workload), which
+// are searched there.
+constexpr uint32_t kRelocLines = 8;   // lines in flight per quad
 
-__global__ __launch_bounds__(kRelocThreads) void k_reloc(RelocDev R, const uint64_t* in, uint64_t* out, uint64_t n,
-                                                         int vec) {
-  constexpr uint32_t kW = 2 * kRelocPairs;  // words per lane per chunk
-  __shared__ uint64_t s_q[kRelocThreads / 64][64 * kW];
-  const uint64_t chunk = (uint64_t)kRelocThreads * kRelocPairs;
+template <bool kRooted, uint32_t kPairs>
+__global__ __launch_bounds__(kRelocThreads) void k_reloc(RelocDev R, const uint64_t* in, uint64_t* out, uint64_t n) {
+  constexpr uint32_t kLines = kPairs > 1 ? kRelocLines : 2;
+  __shared__ u64x2 s_w[kRelocThreads / 64][64 * kPairs];
+  __shared__ uint16_t s_pos[kRelocThreads / 64][128 * kPairs];
+  __shared__ uint2 s_lx[kRelocThreads / 64][kSearchBatch];
+  const uint64_t chunk = (uint64_t)kRelocThreads * kPairs;
   const uint32_t lane = threadIdx.x & 63;
-  const uint64_t lt = (1ull << lane) - 1;
-  uint64_t* sq = s_q[threadIdx.x >> 6];
-  if (vec) {
-    const uint64_t pairs = n / 2;
-    const ulonglong2* in2 = reinterpret_cast<const ulonglong2*>(in);
-    ulonglong2* out2 = reinterpret_cast<ulonglong2*>(out);
-    for (uint64_t c = (uint64_t)blockIdx.x * chunk; c < pairs; c += (uint64_t)gridDim.x * chunk) {
-      uint64_t w[kW];
+  u64x2* sp = s_w[threadIdx.x >> 6];
+  uint64_t* sw = reinterpret_cast<uint64_t*>(sp);
+  uint16_t* pos = s_pos[threadIdx.x >> 6];
+  const uint64_t pairs = n / 2;
+  const u64x2a8* in2 = reinterpret_cast<const u64x2a8*>(in);
+  u64x2a8* out2 = reinterpret_cast<u64x2a8*>(out);
+  auto load = [&](uint64_t c, u64x2a8* v) {
 #pragma unroll
-      for (uint32_t q = 0; q < kRelocPairs; ++q) {
-        const uint64_t p = c + q * kRelocThreads + threadIdx.x;
-        const ulonglong2 v = p < pairs ? in2[p] : ulonglong2{0, 0};
-        w[2 * q] = v.x;
-        w[2 * q + 1] = v.y;
-      }
-      uint32_t need = 0, rank[kW], cnt = 0;
-      if (R.n != 0) {
-#pragma unroll
-        for (uint32_t j = 0; j < kW; ++j)
-          if (w[j] >= R.lo_min && (R.policy ? w[j] <= R.hi_max : w[j] < R.hi_max)) need |= 1u << j;
-      }
-#pragma unroll
-      for (uint32_t j = 0; j < kW; ++j) {
-        const uint64_t mk = __ballot((need >> j) & 1);
-        rank[j] = cnt + (uint32_t)__popcll(mk & lt);
-        if ((need >> j) & 1) sq[rank[j]] = w[j];
-        cnt += (uint32_t)__popcll(mk);
-      }
-      // The wave's own LDS words: its writes precede its reads in program order.
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      for (uint32_t b = 0; b < cnt; b += 64 * kRelocSearch) {
-        uint64_t x[kRelocSearch], y[kRelocSearch];
-        uint32_t mm = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < kRelocSearch; ++k) {
-          const uint32_t i = b + 64 * k + lane;
-          x[k] = i < cnt ? sq[i] : 0;
-          mm |= (i < cnt ? 1u : 0u) << k;
-        }
-        reloc_batch<kRelocSearch>(R, x, y, mm);
-#pragma unroll
-        for (uint32_t k = 0; k < kRelocSearch; ++k) {
-          const uint32_t i = b + 64 * k + lane;
-          if (i < cnt) sq[i] = y[k];
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (uint32_t j = 0; j < kW; ++j)
-        if ((need >> j) & 1) w[j] = sq[rank[j]];
-#pragma unroll
-      for (uint32_t q = 0; q < kRelocPairs; ++q) {
-        const uint64_t p = c + q * kRelocThreads + threadIdx.x;
-        if (p < pairs) out2[p] = ulonglong2{w[2 * q], w[2 * q + 1]};
-      }
-      // The next chunk's compaction overwrites this wave's LDS words only
-      // after every lane has read its own back (program order in the wave).
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (uint32_t q = 0; q < kPairs; ++q) {
+      const uint64_t p = c + q * kRelocThreads + threadIdx.x;
+      v[q] = p < pairs ? in2[p] : u64x2a8{0, 0};
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0 && (n & 1)) out[n - 1] = reloc_word(R, in[n - 1]);
-  } else {
-    const uint64_t stride = (uint64_t)gridDim.x * kRelocThreads;
-    for (uint64_t p = (uint64_t)blockIdx.x * kRelocThreads + threadIdx.x; p < n; p += stride)
-      out[p] = reloc_word(R, in[p]);
+  };
+  u64x2a8 v[kPairs];
+  load((uint64_t)blockIdx.x * chunk, v);
+  for (uint64_t c = (uint64_t)blockIdx.x * chunk; c < pairs; c += (uint64_t)gridDim.x * chunk) {
+    if (R.n > 1) {
+      uint32_t cnt = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < kPairs; ++q) {
+        const bool n0 = reloc_in_range(R, v[q].x), n1 = reloc_in_range(R, v[q].y);
+        const uint64_t m0 = __ballot(n0), m1 = __ballot(n1);
+        sp[64 * q + lane] = u64x2{v[q].x, v[q].y};
+        if (n0) pos[cnt + lanes_below(m0)] = (uint16_t)(128 * q + 2 * lane);
+        cnt += (uint32_t)__popcll(m0);
+        if (n1) pos[cnt + lanes_below(m1)] = (uint16_t)(128 * q + 2 * lane + 1);
+        cnt += (uint32_t)__popcll(m1);
+      }
+      load(c + (uint64_t)gridDim.x * chunk, v);
+      wave_search<kLines, kRooted>(R, sw, pos, s_lx[threadIdx.x >> 6], cnt);
+#pragma unroll
+      for (uint32_t q = 0; q < kPairs; ++q) {
+        const uint64_t p = c + q * kRelocThreads + threadIdx.x;
+        const u64x2 r = sp[64 * q + lane];
+        if (p < pairs) st_stream(out2 + p, u64x2a8{r.x, r.y});
+      }
+      wave_fence();  // the next chunk's words follow every lane's reads
+    } else {
+      u64x2a8 r[kPairs];
+#pragma unroll
+      for (uint32_t q = 0; q < kPairs; ++q) r[q] = u64x2a8{reloc_word(R, v[q].x), reloc_word(R, v[q].y)};
+      load(c + (uint64_t)gridDim.x * chunk, v);
+#pragma unroll
+      for (uint32_t q = 0; q < kPairs; ++q) {
+        const uint64_t p = c + q * kRelocThreads + threadIdx.x;
+        if (p < pairs) st_stream(out2 + p, r[q]);
+      }
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && (n & 1)) {
+    uint64_t o = in[n - 1];
+    if constexpr (kRooted) {
+      o = reloc_word(R, o);
+    } else {
+      const uint64_t w = o;
+      reloc_batch<1>(R, &w, &o, 1u);
+    }
+    out[n - 1] = o;
   }
 }
 
@@ -2802,7 +3033,7 @@ hipError_t launch_index_count(const IndexArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_index_count, dim3((uint32_t)nblocks), dim3(kIndexThreads), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_index_scan, dim3(1), dim3(kIndexScanThreads), 0, s, a, nblocks);
+  hipLaunchKernelGGL(k_index_scan, dim3(1), dim3(kIndexScanThreads), 0, s, a, nblocks, a.nb);
   return hipGetLastError();
 }
 
@@ -2813,13 +3044,31 @@ hipError_t launch_index_place(const IndexArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t launch_roots_count(const IndexArgs& a, hipStream_t s) {
+  const uint64_t nblocks = (a.nb + kRootBlock - 1) / kRootBlock;
+  if (nblocks == 0 || nblocks > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_roots_count, dim3((uint32_t)nblocks), dim3(kRootBlock), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_index_scan, dim3(1), dim3(kIndexScanThreads), 0, s, a, nblocks, 1ull);  // after line 0
+  return hipGetLastError();
+}
+
+hipError_t launch_roots_place(const IndexArgs& a, hipStream_t s) {
+  const uint64_t nblocks = (a.nb + kRootBlock - 1) / kRootBlock;
+  if (nblocks == 0 || nblocks > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_roots_place, dim3((uint32_t)nblocks), dim3(kRootBlock), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_reloc_words(const RelocDev& r, const uint64_t* in, uint64_t* out, uint64_t n, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  const int vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-  const uint64_t per_block = (uint64_t)kRelocThreads * (vec ? 2 * kRelocPairs : 1);
-  uint64_t blocks = (n + per_block - 1) / per_block;
-  if (blocks > 256 * 32) blocks = 256 * 32;
-  hipLaunchKernelGGL(k_reloc, dim3((uint32_t)blocks), dim3(kRelocThreads), 0, s, r, in, out, n, vec);
+  const bool few = n <= kRelocFewWords, rooted = r.root || r.n <= 1;
+  const uint64_t per_block = (uint64_t)kRelocThreads * 2 * (few ? 1 : kRelocPairs);
+  const dim3 blocks((uint32_t)std::min<uint64_t>((n + per_block - 1) / per_block, kRelocBlocks));
+  const auto kernel = rooted ? (few ? k_reloc<true, 1> : k_reloc<true, kRelocPairs>)
+                             : (few ? k_reloc<false, 1> : k_reloc<false, kRelocPairs>);
+  hipLaunchKernelGGL(kernel, blocks, dim3(kRelocThreads), 0, s, r, in, out, n);
   return hipGetLastError();
 }
 

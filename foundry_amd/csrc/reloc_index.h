@@ -1,9 +1,11 @@
-// reloc_index.h -- the interval index of the relocation search and its
-// builder.  The builder's per-root-line steps are host and device code
-// alike: the library builds relocation plans and an archive's index with
-// them as kernels (one thread per root line, kernels.hip), the no-allocation
-// entry point and the CPU check of the search (tests/native) on the host,
-// so both produce the same lines.
+// reloc_index.h -- the interval indexes of the relocation search and their
+// builders, whose steps are host and device code alike.  The two-level index
+// (root entries over leaf lines) serves archives and relocation plans and is
+// built by kernels (kernels.hip), a thread per root entry and per line; the
+// index of root lines serves the no-allocation entry point (built on the
+// host) and is what a plan is inspected by (built by kernels).  The CPU
+// checks (tests/native) build both on the host, so both sides produce the
+// same lines.
 #pragma once
 
 #include <stdint.h>
@@ -29,10 +31,8 @@ struct HostIndex {
 // Root lines per interval, about (between k/2 and k per interval, a power
 // of two in all): a root line whose range holds more than four intervals
 // takes a second read, its child.  More root lines mean fewer second reads
-// and a larger index (64 B per line): 2 per interval for the index that
-// lives beside a restored archive, 16 for a relocation plan, which is built
-// once to relocate many words (2M intervals: 1.55 reads per lookup and
-// 228 MB, against about 1.3 reads and 2 GB).
+// and a larger index (64 B per line): 2 per interval for the no-allocation
+// entry point's index, 16 for the lines a relocation plan is inspected by.
 constexpr uint64_t kRootLinesPerInterval = 2;
 constexpr uint64_t kPlanRootLinesPerInterval = 16;
 constexpr uint32_t kLeafIntervals = kLineSlots;  // the interval at or before B, and three starting inside
@@ -44,24 +44,27 @@ struct IndexShape {
   uint64_t nb;
 };
 
-// Checks a table (sorted, non-overlapping, non-empty intervals below 2^64-1
-// spanning less than 2^54 bytes, fewer than 2^32 of them) and picks the
-// root lines: the line width is the smallest power of two giving at most
-// `target` root lines over [lo_min, hi_max], and at most 2^31 so offsets
-// inside a line fit in 31 bits (a span of 2^47, a process's whole address
-// space, then takes at most 2^16 root lines).
-inline int index_shape(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint64_t n, uint32_t policy,
-                       uint64_t root_lines_per_interval, IndexShape* shape, std::string* why) {
+// Checks a table: sorted, non-overlapping, non-empty intervals below 2^64-1
+// spanning less than 2^54 bytes, fewer than 2^32 of them.  *off_bits gets
+// the OR of every lo - lo[0] (the starts' common alignment).
+inline int check_table(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint64_t n, uint32_t policy,
+                       uint64_t* off_bits, std::string* why) {
   auto err = [why](int code, const std::string& msg) {
     *why = msg;
     return code;
   };
+  *off_bits = 0;
   if (policy > FDY_RELOC_INCLUSIVE) return err(FDY_E_INVALID, "unknown relocation policy");
-  shape->shift = 0;
-  shape->nb = 0;
   if (n == 0) return FDY_OK;
   if (!lo || !hi || !nlo) return err(FDY_E_INVALID, "null interval array");
-  for (uint64_t i = 0; i < n; ++i) {
+  // One pass without branches (every LOAD pays for it); a table that fails
+  // is walked again for the first interval at fault.
+  uint64_t bits = 0, bad = (uint64_t)(lo[0] >= hi[0]) | (uint64_t)(hi[0] == UINT64_MAX);
+  for (uint64_t i = 1; i < n; ++i) {
+    bad |= (uint64_t)(lo[i] >= hi[i]) | (uint64_t)(hi[i] == UINT64_MAX) | (uint64_t)(hi[i - 1] > lo[i]);
+    bits |= lo[i] - lo[0];
+  }
+  for (uint64_t i = 0; bad && i < n; ++i) {
     if (lo[i] >= hi[i]) return err(FDY_E_INVALID, "interval " + std::to_string(i) + " is empty (lo >= hi)");
     if (hi[i] == UINT64_MAX) return err(FDY_E_INVALID, "interval " + std::to_string(i) + " ends at 2^64-1");
     if (i && hi[i - 1] > lo[i])
@@ -69,16 +72,29 @@ inline int index_shape(const uint64_t* lo, const uint64_t* hi, const uint64_t* n
                                     " overlap or are not sorted by lo");
   }
   if (n > 0xFFFFFFF0ull) return err(FDY_E_INVALID, "more than 2^32 intervals");
-  const uint64_t span = hi[n - 1] - lo[0];
-  if (span >> 54) return err(FDY_E_INVALID, "intervals span more than 2^54 bytes");
+  if ((hi[n - 1] - lo[0]) >> 54) return err(FDY_E_INVALID, "intervals span more than 2^54 bytes");
+  *off_bits = bits;
+  return FDY_OK;
+}
+
+// The line width for at most `target` root lines over [lo_min, hi_max]: the
+// smallest power of two, and at most 2^31 so offsets inside a line fit in 31
+// bits (a span of 2^47, a process's whole address space, then takes at most
+// 2^16 root lines).
+inline IndexShape shape_for(uint64_t span, uint64_t target) {
+  IndexShape s{0, 0};
+  while ((span >> s.shift) + 1 > target) ++s.shift;
+  if (s.shift > kMaxLineShift) s.shift = kMaxLineShift;
+  s.nb = (span >> s.shift) + 1;  // w - lo_min <= span, so (w - lo_min) >> shift < nb
+  return s;
+}
+
+// The root lines of a checked table of n intervals over `span` bytes, at most
+// `root_lines_per_interval` per interval rounded up to a power of two in all.
+inline IndexShape line_shape(uint64_t span, uint64_t n, uint64_t root_lines_per_interval) {
   uint64_t target = 1;
   while (target < root_lines_per_interval * n) target <<= 1;
-  uint32_t shift = 0;
-  while ((span >> shift) + 1 > target) ++shift;
-  if (shift > kMaxLineShift) shift = kMaxLineShift;
-  shape->shift = shift;
-  shape->nb = (span >> shift) + 1;  // w - lo_min <= span, so (w - lo_min) >> shift < nb
-  return FDY_OK;
+  return shape_for(span, target);
 }
 
 // First address of root line b.
@@ -174,6 +190,26 @@ __host__ __device__ inline uint64_t subtree_lines(uint64_t m, uint64_t* size, ui
   return total;
 }
 
+// The end field of interval k in a line from s0.
+__host__ __device__ inline uint32_t slot_end(uint64_t s0, uint64_t hi) {
+  if (hi < s0) return 0;
+  const uint64_t e = hi - s0 + 1;
+  return e > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)e;
+}
+
+// A leaf line whose range from s0 holds intervals i
+// (lo[i] <= s0, the last such) .. j.
+__host__ __device__ inline RelocLine leaf_line(uint64_t s0, uint64_t i, uint64_t j, const uint64_t* lo,
+                                               const uint64_t* hi, const uint64_t* nlo) {
+  RelocLine L;
+  L.s[0] = RelocSlot{0, slot_end(s0, hi[i]), nlo[i] - lo[i]};
+  for (uint32_t k = 1; k < kLineSlots; ++k) {
+    if (i + k <= j) L.s[k] = RelocSlot{(uint32_t)(lo[i + k] - s0), slot_end(s0, hi[i + k]), nlo[i + k] - lo[i + k]};
+    else L.s[k] = RelocSlot{kLineNone, 0, 0};
+  }
+  return L;
+}
+
 // The line at `at` whose range from s0 holds intervals i (lo[i] <= s0, the
 // last such) .. j: a leaf for up to four, else a fence line whose children
 // take the next free lines (*next on), each holding until it is placed the
@@ -181,20 +217,9 @@ __host__ __device__ inline uint64_t subtree_lines(uint64_t m, uint64_t* size, ui
 __host__ __device__ inline void place_line(RelocLine* line, uint64_t at, uint64_t s0, uint64_t i, uint64_t j,
                                            const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo,
                                            uint64_t* next) {
-  auto end_of = [&](uint64_t k) -> uint32_t {
-    if (hi[k] < s0) return 0;
-    const uint64_t e = hi[k] - s0 + 1;
-    return e > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)e;
-  };
-  RelocLine L;
   const uint64_t m = j - i + 1;
   if (m <= kLeafIntervals) {
-    L.s[0] = RelocSlot{0, end_of(i), nlo[i] - lo[i]};
-    for (uint32_t k = 1; k < kLineSlots; ++k) {
-      if (i + k <= j) L.s[k] = RelocSlot{(uint32_t)(lo[i + k] - s0), end_of(i + k), nlo[i + k] - lo[i + k]};
-      else L.s[k] = RelocSlot{kLineNone, 0, 0};
-    }
-    line[at] = L;
+    line[at] = leaf_line(s0, i, j, lo, hi, nlo);
     return;
   }
   // A fence line, written field by field in place (a fence array indexed
@@ -233,14 +258,15 @@ __host__ __device__ inline void place_root(RelocLine* line, uint64_t b, uint64_t
   }
 }
 
-// The whole index on the host.
+// The whole index of root lines on the host.
 inline int build_reloc_index(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint64_t n,
                              uint32_t policy, HostIndex* out, std::string* why,
                              uint64_t root_lines_per_interval = kRootLinesPerInterval) {
   std::memset(&out->dev, 0, sizeof(out->dev));
-  IndexShape sh;
-  const int rc = index_shape(lo, hi, nlo, n, policy, root_lines_per_interval, &sh, why);
+  uint64_t off_bits;
+  const int rc = check_table(lo, hi, nlo, n, policy, &off_bits, why);
   if (rc || n == 0) return rc;
+  const IndexShape sh = line_shape(hi[n - 1] - lo[0], n, root_lines_per_interval);
   std::vector<uint64_t> ri(sh.nb), rj(sh.nb), base(sh.nb);
   uint64_t total = sh.nb;
   for (uint64_t b = 0; b < sh.nb; ++b) {
@@ -259,7 +285,184 @@ inline int build_reloc_index(const uint64_t* lo, const uint64_t* hi, const uint6
   out->dev.n = n;
   out->dev.lo_min = lo[0];
   out->dev.hi_max = hi[n - 1];
+  out->dev.span = hi[n - 1] - lo[0] + (policy ? 1 : 0);
+  out->dev.delta = nlo[0] - lo[0];
   out->dev.shift = sh.shift;
+  out->dev.policy = policy;
+  return FDY_OK;
+}
+
+// ---- the two-level index ---------------------------------------------------
+//
+// Root entries over equal address ranges.  An entry inside whose range no
+// interval starts answers by itself; the others name the lines that hold
+// their range's intervals four at a time (RelocRoot).  With 28 intervals or
+// fewer a search is one entry and one leaf line; past that (or past four
+// where the starts are not on the fences' unit) the entry names the top line
+// of a tree of full lines: leaves of four intervals, fence lines of 15
+// children, every level's lines together, the top level first.
+
+constexpr uint64_t kLineKids = kLineFences + 1;
+constexpr uint64_t kRootIntervals = (kRootFences + 1) * kLeafIntervals;
+
+struct RootShape {
+  uint32_t shift, fence_shift;
+  uint64_t nb;
+  bool exact;  // every start lies on a multiple of 2^fence_shift from its entry's first address
+};
+
+// Root entries of a checked table: one to two per interval up to 2^16 (1 MB:
+// with their lines they stay in the L2s), then one per four to eight.  On the
+// relocation workloads' mix of sizes no lookup then meets a tree at 40,000
+// intervals (2% of a 64 GiB archive region's do with a quarter of the entries),
+// 2% at 200,000 and more.  Where the starts' alignment is coarser than 1/2^15
+// of an entry's range, narrower entries (up to four per interval, and up to
+// 32768: 512 KB) make the fences exact.
+inline RootShape root_shape(const uint64_t* lo, const uint64_t* hi, uint64_t n, uint64_t off_bits) {
+  RootShape r{0, 0, 0, true};
+  if (n == 0) return r;
+  const uint64_t span = hi[n - 1] - lo[0];
+  uint64_t t = 1;
+  while (t < 2 * n && (t < (1ull << 16) || 4 * t < n)) t <<= 1;
+  IndexShape s = shape_for(span, t);
+  uint32_t align = 0;  // starts are multiples of 2^align apart
+  while (align < kMaxLineShift && !((off_bits >> align) & 1)) ++align;
+  if (s.shift > kRootFenceBits + align) {
+    const uint64_t nb = (span >> (kRootFenceBits + align)) + 1;
+    if (nb <= std::max<uint64_t>(4 * n, 32768)) s = IndexShape{kRootFenceBits + align, nb};
+  }
+  r.shift = s.shift;
+  r.nb = s.nb;
+  r.fence_shift = s.shift > kRootFenceBits ? s.shift - kRootFenceBits : 0;
+  r.exact = r.fence_shift <= align;
+  return r;
+}
+
+// The first interval of a root entry's range: the last with lo <= s0, its
+// first address, when e intervals start before s0.
+__host__ __device__ inline uint64_t root_first(const uint64_t* lo, uint64_t n, uint64_t s0, uint64_t e) {
+  return e < n && lo[e] == s0 ? e : e - 1;
+}
+
+// Whether m intervals are leaves right below their root entry.
+__host__ __device__ inline bool root_flat(uint64_t m, bool exact) {
+  return m <= kLeafIntervals || (exact && m <= kRootIntervals);
+}
+
+// Lines below a root entry whose range holds m intervals (the last one
+// starting at or before its first address among them).
+__host__ __device__ inline uint64_t root_lines(uint64_t m, bool exact) {
+  if (m == 1) return 0;  // a direct entry
+  uint64_t w = kLeafIntervals, total = (m + w - 1) / w;
+  if (root_flat(m, exact)) return total;
+  while (w < m) {
+    w *= kLineKids;
+    total += (m + w - 1) / w;
+  }
+  return total;
+}
+
+// The root entry from s0 whose range holds intervals i .. j, its lines from
+// line `first` on.
+__host__ __device__ inline RelocRoot root_entry(uint64_t s0, uint64_t i, uint64_t j, const uint64_t* lo,
+                                                const uint64_t* hi, const uint64_t* nlo, uint32_t fence_shift,
+                                                bool exact, uint64_t first) {
+  RelocRoot r;
+  if (i == j) {
+    const uint64_t delta = nlo[i] - lo[i];
+    r.line = kRootDirect;
+    r.word[0] = slot_end(s0, hi[i]);
+    r.word[1] = (uint32_t)delta;
+    r.word[2] = (uint32_t)(delta >> 32);
+    return r;
+  }
+  const bool flat = root_flat(j - i + 1, exact);
+  r.line = (uint32_t)first | (flat ? 0u : kRootTree);
+  for (uint32_t e = 0; e < kRootFences / 2; ++e) {
+    uint32_t f[2];
+    for (uint32_t h = 0; h < 2; ++h) {
+      const uint64_t k = i + (uint64_t)(2 * e + h + 1) * kLeafIntervals;
+      f[h] = flat && k <= j ? (uint32_t)((lo[k] - s0) >> fence_shift) : 0xFFFFu;
+    }
+    r.word[e] = f[0] | (f[1] << 16);
+  }
+  return r;
+}
+
+// Line 0, a leaf that moves nothing.
+__host__ __device__ inline RelocLine null_line() {
+  RelocLine L;
+  L.s[0] = RelocSlot{0, 0, 0};
+  for (uint32_t k = 1; k < kLineSlots; ++k) L.s[k] = RelocSlot{kLineNone, 0, 0};
+  return L;
+}
+
+// Line k of the root_lines() lines (the first at `first`) below an entry
+// whose range from s0 holds intervals i .. j.
+__host__ __device__ inline void place_below(RelocLine* line, uint64_t first, uint64_t k, uint64_t s0, uint64_t i,
+                                            uint64_t j, const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo,
+                                            bool exact) {
+  const uint64_t m = j - i + 1;
+  // The level holding line k: intervals per line, its first line, its lines.
+  uint64_t w = kLeafIntervals, at = 0, size = 0;
+  if (!root_flat(m, exact)) {
+    while (w < m) w *= kLineKids;
+    for (;; w /= kLineKids) {
+      size = (m + w - 1) / w;
+      if (k < at + size) break;
+      at += size;
+    }
+  }
+  const uint64_t a = i + (k - at) * w;          // the line's first interval
+  const uint64_t B = k == at ? s0 : lo[a];      // and first address
+  const uint64_t z = j - a < w ? j : a + w - 1; // its last interval
+  if (w == kLeafIntervals) {
+    line[first + k] = leaf_line(B, a, z, lo, hi, nlo);
+    return;
+  }
+  const uint64_t cw = w / kLineKids;  // intervals per child
+  uint32_t* L = reinterpret_cast<uint32_t*>(line + first + k);
+  L[0] = kLineFence;
+  L[1] = (uint32_t)(first + at + size + (k - at) * kLineKids);
+  for (uint32_t e = 0; e < kLineFences; ++e) {
+    const uint64_t c = a + (e + 1) * cw;
+    L[2 + e] = c <= z ? (uint32_t)(lo[c] - B) : kLineNone;
+  }
+}
+
+// The whole two-level index on the host (what the device build is held to).
+struct HostRootIndex {
+  std::vector<RelocRoot> root;
+  std::vector<RelocLine> line;
+  RelocDev dev{};
+};
+inline int build_root_index(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint64_t n, uint32_t policy,
+                            HostRootIndex* out, std::string* why) {
+  std::memset(&out->dev, 0, sizeof(out->dev));
+  uint64_t off_bits;
+  const int rc = check_table(lo, hi, nlo, n, policy, &off_bits, why);
+  if (rc || n == 0) return rc;
+  const RootShape sh = root_shape(lo, hi, n, off_bits);
+  out->root.resize(sh.nb);
+  out->line.assign(1, null_line());
+  uint64_t e = 0;
+  for (uint64_t b = 0; b < sh.nb; ++b) {
+    const uint64_t s0 = root_start(lo[0], sh.shift, b), s1 = root_start(lo[0], sh.shift, b + 1);
+    const uint64_t i = root_first(lo, n, s0, e);
+    while (e < n && lo[e] < s1) ++e;
+    const uint64_t first = out->line.size(), below = root_lines(e - i, sh.exact);
+    out->root[b] = root_entry(s0, i, e - 1, lo, hi, nlo, sh.fence_shift, sh.exact, first);
+    out->line.resize(first + below);
+    for (uint64_t k = 0; k < below; ++k)
+      place_below(out->line.data(), first, k, s0, i, e - 1, lo, hi, nlo, sh.exact);
+  }
+  out->dev.n = n;
+  out->dev.lo_min = lo[0];
+  out->dev.hi_max = hi[n - 1];
+  out->dev.span = hi[n - 1] - lo[0] + (policy ? 1 : 0);
+  out->dev.delta = nlo[0] - lo[0];
+  out->dev.shift = sh.shift;
+  out->dev.fence_shift = sh.fence_shift;
   out->dev.policy = policy;
   return FDY_OK;
 }

@@ -194,23 +194,91 @@ int build_reloc_index(const uint64_t* lo, const uint64_t* hi, const uint64_t* nl
   return rc ? err(rc, why) : FDY_OK;
 }
 
-// A table's index on the device: checked and shaped on the host, its lines
-// counted, placed and written on the device (one thread per root line,
-// kernels.hip), so only the table travels over PCIe.  Synchronizes.
+// The index of root lines of the table at ia.lo, ia.hi, ia.nlo (device
+// memory; a checked table): *total lines, at `out` unless out is null.
+// Synchronizes.
+int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interval, DevBuf* out, uint64_t* total,
+                     uint32_t* shift) {
+  const IndexShape sh = line_shape(span, ia.n, root_lines_per_interval);
+  *shift = sh.shift;
+  const uint64_t nblocks = (sh.nb + kIndexThreads - 1) / kIndexThreads;
+  DevBuf sums;
+  int rc = dev_alloc(sums, 8 * (nblocks + 1), "interval index counts");
+  if (rc) return rc;
+  ia.nb = sh.nb;
+  ia.shift = sh.shift;
+  ia.block_sum = sums.as<uint64_t>();
+  ia.total = sums.as<uint64_t>() + nblocks;
+  FDY_HIP(launch_index_count(ia, nullptr));
+  FDY_HIP(hipMemcpy(total, ia.total, 8, hipMemcpyDeviceToHost));
+  if (*total > kMaxIndexLines) return err(FDY_E_INVALID, "interval index too large");
+  if (!out) return FDY_OK;
+  rc = dev_alloc(*out, *total * sizeof(RelocLine), "interval index lines");
+  if (rc) return rc;
+  ia.line = out->as<RelocLine>();
+  FDY_HIP(launch_index_place(ia, nullptr));
+  FDY_HIP(hipStreamSynchronize(nullptr));  // before the counts (and a caller's table) are freed
+  return FDY_OK;
+}
+
+// A table's two-level index on the device: its lines counted, placed and
+// written there, root entries first in `out`.  Synchronizes.
+int place_roots(IndexArgs ia, const RootShape& sh, DevBuf* out, RelocDev* dev) {
+  const uint64_t nblocks = (sh.nb + kRootBlock - 1) / kRootBlock;
+  DevBuf work;
+  int rc = dev_alloc(work, 8 * (nblocks + 1) + 4 * sh.nb, "interval index counts");
+  if (rc) return rc;
+  ia.nb = sh.nb;
+  ia.shift = sh.shift;
+  ia.fence_shift = sh.fence_shift;
+  ia.exact = sh.exact;
+  ia.block_sum = work.as<uint64_t>();
+  ia.total = work.as<uint64_t>() + nblocks;
+  ia.ends = reinterpret_cast<uint32_t*>(work.as<uint64_t>() + nblocks + 1);
+  FDY_HIP(launch_roots_count(ia, nullptr));
+  uint64_t total = 0;
+  FDY_HIP(hipMemcpy(&total, ia.total, 8, hipMemcpyDeviceToHost));
+  if (total > kRootDirect) return err(FDY_E_INVALID, "interval index too large");
+  const uint64_t root_bytes = (sh.nb * sizeof(RelocRoot) + 255) / 256 * 256;
+  rc = dev_alloc(*out, root_bytes + total * sizeof(RelocLine), "interval index");
+  if (rc) return rc;
+  dev->root = ia.root = out->as<RelocRoot>();
+  dev->line = ia.line = reinterpret_cast<RelocLine*>(out->as<uint8_t>() + root_bytes);
+  dev->shift = sh.shift;
+  dev->fence_shift = sh.fence_shift;
+  FDY_HIP(launch_roots_place(ia, nullptr));
+  FDY_HIP(hipStreamSynchronize(nullptr));  // before the counts (and a caller's table) are freed
+  return FDY_OK;
+}
+
+// Plans of more intervals keep an index of root lines.  Their root entries
+// and lines no longer stay in the L2s, and a lookup then costs 1.4 reads that
+// miss them, against 1.24 in an index of 16 root lines per interval: 32M words
+// relocate in 251 us (two-level) and 259 us (root lines) at 700,000
+// intervals, 280 and 264 us at a million, 202 and 246 us at 400,000.
+constexpr uint64_t kRootedIntervals = 3ull << 18;
+
+// The index of a table checked and shaped on the host, built on the device
+// (only the table travels over PCIe).  A table is refused when its index of
+// `root_lines_per_interval` root lines has more than 32 bits can name.
+// plan: the device copy of the table stays (at out->table) for
+// fdy_reloc_plan_lines, unless the plan's own index is those lines.  Synchronizes.
 int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint64_t n, uint32_t policy,
-                     RelocPlan* out, uint64_t root_lines_per_interval = kRootLinesPerInterval) {
+                     RelocPlan* out, uint64_t root_lines_per_interval, bool plan) {
   std::memset(&out->dev, 0, sizeof(out->dev));
-  out->line.release();
+  out->index.release();
+  out->table.release();
   std::string why;
-  IndexShape sh;
-  int rc = index_shape(lo, hi, nlo, n, policy, root_lines_per_interval, &sh, &why);
+  uint64_t off_bits;
+  int rc = check_table(lo, hi, nlo, n, policy, &off_bits, &why);
   if (rc) return err(rc, why);
   out->dev.policy = policy;
   if (n == 0) return FDY_OK;
-  const uint64_t nblocks = (sh.nb + kIndexThreads - 1) / kIndexThreads;
-  DevBuf table, sums;
+  const uint64_t span = hi[n - 1] - lo[0];
+  if (line_shape(span, n, root_lines_per_interval).nb > kMaxIndexLines)
+    return err(FDY_E_INVALID, "interval index too large");
+  DevBuf table;
   rc = dev_alloc(table, 24 * n, "interval table");
-  if (!rc) rc = dev_alloc(sums, 8 * (nblocks + 1), "interval index counts");
   if (rc) return rc;
   uint64_t* t = table.as<uint64_t>();
   FDY_HIP(hipMemcpy(t, lo, 8 * n, hipMemcpyHostToDevice));
@@ -221,24 +289,24 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
   ia.hi = t + n;
   ia.nlo = t + 2 * n;
   ia.n = n;
-  ia.nb = sh.nb;
-  ia.shift = sh.shift;
-  ia.block_sum = sums.as<uint64_t>();
-  ia.total = sums.as<uint64_t>() + nblocks;
-  FDY_HIP(launch_index_count(ia, nullptr));
-  uint64_t total = 0;
-  FDY_HIP(hipMemcpy(&total, ia.total, 8, hipMemcpyDeviceToHost));
-  if (total > kMaxIndexLines) return err(FDY_E_INVALID, "interval index too large");
-  rc = dev_alloc(out->line, total * sizeof(RelocLine), "interval index lines");
+  RelocDev d = out->dev;
+  if (n == 1) {  // one delta: no index
+    if (plan) out->table.swap(table);
+  } else if (plan && n > kRootedIntervals) {
+    uint64_t total = 0;
+    rc = place_root_lines(ia, span, root_lines_per_interval, &out->index, &total, &d.shift);
+    d.line = out->index.as<RelocLine>();
+  } else {
+    rc = place_roots(ia, root_shape(lo, hi, n, off_bits), &out->index, &d);
+    if (plan) out->table.swap(table);
+  }
   if (rc) return rc;
-  ia.line = out->line.as<RelocLine>();
-  FDY_HIP(launch_index_place(ia, nullptr));
-  FDY_HIP(hipStreamSynchronize(nullptr));  // before the table and counts are freed
-  out->dev.line = out->line.as<RelocLine>();
-  out->dev.n = n;
-  out->dev.lo_min = lo[0];
-  out->dev.hi_max = hi[n - 1];
-  out->dev.shift = sh.shift;
+  d.n = n;
+  d.lo_min = lo[0];
+  d.hi_max = hi[n - 1];
+  d.span = span + (policy ? 1 : 0);
+  d.delta = nlo[0] - lo[0];
+  out->dev = d;
   return FDY_OK;
 }
 
@@ -466,7 +534,7 @@ int compact_for_serving(fdy_archive* a, hipStream_t s) {
 
 uint64_t held_bytes(const fdy_archive* a) {
   const DevBuf* bufs[] = {&a->arena, &a->img, &a->image, &a->aux, &a->live, &a->ovr, &a->cand,
-                          &a->reloc.line};
+                          &a->reloc.index};
   uint64_t n = 0;
   for (const DevBuf* b : bufs) n += b->bytes;
   return n;
@@ -845,7 +913,7 @@ int fdy_archive_set_relocation(fdy_archive* a, const uint64_t* lo, const uint64_
   FDY_HIP(hipDeviceSynchronize());  // kernels in flight may still read the old table
   a->reloc.~RelocPlan();
   new (&a->reloc) RelocPlan();
-  return build_reloc_plan(lo, hi, nlo, n, policy, &a->reloc);
+  return build_reloc_plan(lo, hi, nlo, n, policy, &a->reloc, kRootLinesPerInterval, false);
 }
 
 int fdy_archive_set_groups(fdy_archive* a, const uint32_t* template_of) {
@@ -1429,7 +1497,7 @@ int fdy_reloc_plan_create(const uint64_t* lo, const uint64_t* hi, const uint64_t
   if (!out) return err(FDY_E_INVALID, "null output");
   auto p = std::make_unique<fdy_reloc_plan>();
   (void)hipGetDevice(&p->device);
-  int rc = build_reloc_plan(lo, hi, nlo, n, policy, &p->plan, kPlanRootLinesPerInterval);
+  int rc = build_reloc_plan(lo, hi, nlo, n, policy, &p->plan, kPlanRootLinesPerInterval, true);
   if (rc) return rc;
   *out = p.release();
   return FDY_OK;
@@ -1437,13 +1505,30 @@ int fdy_reloc_plan_create(const uint64_t* lo, const uint64_t* hi, const uint64_t
 
 int fdy_reloc_plan_lines(const fdy_reloc_plan* p, void* lines, uint64_t cap, uint64_t* n_lines) {
   if (!p) return err(FDY_E_INVALID, "null plan");
-  const uint64_t n = p->plan.dev.n ? p->plan.line.bytes / sizeof(RelocLine) : 0;
+  const RelocDev& d = p->plan.dev;
+  uint64_t n = 0;
+  DevBuf built;
+  const void* line = p->plan.index.p;
+  if (d.n && !p->plan.table.p) {
+    n = p->plan.index.bytes / sizeof(RelocLine);
+  } else if (d.n) {
+    FDY_HIP(hipSetDevice(p->device));
+    IndexArgs ia{};
+    ia.lo = p->plan.table.as<uint64_t>();
+    ia.hi = ia.lo + d.n;
+    ia.nlo = ia.lo + 2 * d.n;
+    ia.n = d.n;
+    uint32_t shift = 0;
+    const int rc = place_root_lines(ia, d.hi_max - d.lo_min, kPlanRootLinesPerInterval, lines ? &built : nullptr, &n, &shift);
+    if (rc) return rc;
+    line = built.p;
+  }
   if (n_lines) *n_lines = n;
   if (!lines) return FDY_OK;
   if (cap < n) return err(FDY_E_CAPACITY, "output holds " + std::to_string(cap) + " lines, the index has " +
                                               std::to_string(n));
   FDY_HIP(hipSetDevice(p->device));
-  if (n) FDY_HIP(hipMemcpy(lines, p->plan.line.p, n * sizeof(RelocLine), hipMemcpyDeviceToHost));
+  if (n) FDY_HIP(hipMemcpy(lines, line, n * sizeof(RelocLine), hipMemcpyDeviceToHost));
   return FDY_OK;
 }
 

@@ -148,7 +148,8 @@ struct NodeDesc {
 };
 static_assert(sizeof(NodeDesc) == 32, "NodeDesc is 32 B");
 
-// The interval index: 64-byte lines, each answering every search inside
+// The interval index of root lines (the no-allocation entry point's, and
+// the one a plan is inspected by): 64-byte lines, each answering every search inside
 // its address range from that one line or naming the line that does.  Root
 // line b covers addresses [lo_min + b*2^shift, lo_min + (b+1)*2^shift)
 // (shift <= 31, so offsets inside a line fit in 31 bits).
@@ -184,13 +185,39 @@ static_assert(sizeof(RelocLine) == 64, "RelocLine is one 64-byte line");
 // Fence f of a fence line: its 32-bit word 2 + f.
 __host__ __device__ inline uint32_t* line_fences(RelocLine& L) { return reinterpret_cast<uint32_t*>(&L) + 2; }
 
+// The two-level index (archives and relocation plans): lines as above, but
+// under root entries of 16 bytes.  A root entry covers the 2^shift addresses
+// from lo_min + b * 2^shift on.  Where no interval starts inside its range it
+// answers itself (kRootDirect): its other words are the end and the delta of
+// the interval before it, as in a slot (end 0: that interval does not reach
+// it).  Otherwise the leaf lines line .. line + 6 hold the range's intervals
+// (as many as it has fences, and one), child c starting at fence c - 1 (child
+// 0 at the entry's first address), or (kRootTree) the fence line at the top
+// of a tree whose descent goes on as above.  A fence is an offset inside the
+// entry's range in units of 2^fence_shift, below 2^15 (unused: 0xFFFF).  Line
+// 0 moves nothing: a search through a direct entry ends there.
+constexpr uint32_t kRootFences = 6;
+constexpr uint32_t kRootFenceBits = 15;
+constexpr uint32_t kRootTree = 0x80000000u;
+constexpr uint32_t kRootDirect = 0x40000000u;  // also the line count's limit
+struct RelocRoot {
+  uint32_t line;     // | kRootTree, or kRootDirect
+  uint32_t word[3];  // fences, the first in the low half of word 0; or end, delta
+};
+static_assert(sizeof(RelocRoot) == 16, "a root entry is one 16-byte load");
+
 struct RelocDev {
-  const RelocLine* line;
+  const RelocLine* line;  // root lines first, or (root not null) the two-level index's lines
+  const RelocRoot* root;  // two-level index
   uint64_t n;           // intervals; 0 = relocation off
   uint64_t lo_min;
   uint64_t hi_max;
+  uint64_t span;        // addresses from lo_min that the table can move: hi_max - lo_min (+ 1: inclusive)
+  uint64_t delta;       // new_lo - lo of the first interval (all there is to know when n == 1)
   uint32_t shift;       // <= kMaxLineShift
   uint32_t policy;
+  uint32_t fence_shift; // unit of the root entries' fences
+  uint32_t pad_;
 };
 
 __device__ inline uint32_t ld_u32(const uint8_t* p) {
@@ -227,11 +254,17 @@ __device__ __forceinline__ uint64_t f64(const uint8_t* e, uint32_t off) {
   return (uint64_t)f32(e, off) | ((uint64_t)f32(e, off + 4) << 32);
 }
 
+// Whether w lies inside the table's range (a word outside it is no saved
+// pointer).
+__host__ __device__ __forceinline__ bool reloc_in_range(const RelocDev& r, uint64_t w) {
+  return w - r.lo_min < r.span;
+}
+
 // Relocate K words at once (the words whose bit is set in `mask`; the others
-// pass through): the interval containing w (the last one with lo <= w)
-// moves w if w < hi (w <= hi under the inclusive policy).  The K searches
-// advance in lockstep, so each step issues its K line reads before waiting
-// for any of them.
+// pass through) through an index of root lines: the interval containing w
+// (the last one with lo <= w) moves w if w < hi (w <= hi under the inclusive
+// policy).  The K searches advance in lockstep, so each step issues its K
+// line reads before waiting for any of them.
 template <int K>
 __host__ __device__ inline void reloc_batch(const RelocDev& r, const uint64_t* w, uint64_t* out, uint32_t mask) {
   if (r.n == 0) {  // relocation off (uniform)
@@ -248,7 +281,7 @@ __host__ __device__ inline void reloc_batch(const RelocDev& r, const uint64_t* w
   // go one after another instead of together.
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    ok[k] = ((mask >> k) & 1) && w[k] >= r.lo_min && (r.policy ? w[k] <= r.hi_max : w[k] < r.hi_max);
+    ok[k] = ((mask >> k) & 1) && reloc_in_range(r, w[k]);
     const uint64_t rel = w[k] - r.lo_min;
     const uint64_t b = ok[k] ? rel >> r.shift : 0;
     x[k] = ok[k] ? (uint32_t)(rel - (b << r.shift)) : 0u;
@@ -300,10 +333,69 @@ __host__ __device__ inline void reloc_batch(const RelocDev& r, const uint64_t* w
   }
 }
 
+// The line under root entry rt (its leaf, its tree's top, or line 0 for a
+// direct entry) that holds offset *x of the entry's range; *x becomes the
+// offset inside that line.
+__host__ __device__ __forceinline__ uint32_t root_child(const uint4& rt, uint32_t fence_shift, uint32_t* x) {
+  const uint32_t u = *x >> fence_shift;
+  const uint32_t f[kRootFences / 2] = {rt.y, rt.z, rt.w};
+  uint32_t c = 0, at = 0;
+#pragma unroll
+  for (uint32_t e = 0; e < kRootFences / 2; ++e) {
+    const uint32_t f0 = f[e] & 0xFFFFu, f1 = f[e] >> 16;
+    c += (f0 <= u) + (f1 <= u);
+    at = f0 <= u ? f0 : at;
+    at = f1 <= u ? f1 : at;
+  }
+  if (rt.x & kRootDirect) return 0;
+  *x -= at << fence_shift;
+  return (rt.x & ~kRootTree) + c;
+}
+
+// Whether offset x lies inside an interval with this end field.
+__host__ __device__ __forceinline__ bool slot_holds(const RelocDev& r, uint32_t x, uint32_t end) {
+  return r.policy ? x + 1 <= end : x + 1 < end;
+}
+
+// The leaf under fence line `line` that holds offset *x of it; *x becomes the
+// offset inside the leaf.
+__host__ __device__ __forceinline__ uint32_t tree_leaf(const RelocDev& r, uint32_t line, uint32_t* x) {
+  for (;;) {
+    const uint4* p = reinterpret_cast<const uint4*>(r.line + line);
+    const uint4 v[kLineSlots] = {p[0], p[1], p[2], p[3]};
+    if (!(v[0].x & kLineFence)) return line;
+    const uint32_t f[kLineFences] = {v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w, v[2].x,
+                                     v[2].y, v[2].z, v[2].w, v[3].x, v[3].y, v[3].z, v[3].w};
+    uint32_t c = 0, at = 0;
+#pragma unroll
+    for (uint32_t e = 0; e < kLineFences; ++e) {
+      const bool le = f[e] <= *x;
+      c += le;
+      at = le ? f[e] : at;
+    }
+    *x -= at;
+    line = v[0].y + c;
+  }
+}
+
+// One word through the two-level index, by one lane (the kernels' searches go
+// through wave_search).  A table of one interval (a region moved whole) needs
+// no index: a word in the table's range moves by the one delta.
 __host__ __device__ inline uint64_t reloc_word(const RelocDev& r, uint64_t w) {
-  uint64_t o;
-  reloc_batch<1>(r, &w, &o, 1u);
-  return o;
+  if (r.n == 0 || !reloc_in_range(r, w)) return w;
+  if (r.n == 1) return w + r.delta;
+  const uint64_t rel = w - r.lo_min, b = rel >> r.shift;
+  uint32_t x = (uint32_t)(rel - (b << r.shift));
+  const uint4 rt = *reinterpret_cast<const uint4*>(r.root + b);
+  if (rt.x & kRootDirect) return slot_holds(r, x, rt.y) ? w + ((uint64_t)rt.z | ((uint64_t)rt.w << 32)) : w;
+  uint32_t line = root_child(rt, r.fence_shift, &x);
+  if (rt.x & kRootTree) line = tree_leaf(r, line, &x);
+  const uint32_t* p = reinterpret_cast<const uint32_t*>(r.line + line);
+  uint32_t s = 0;
+#pragma unroll
+  for (uint32_t e = 1; e < kLineSlots; ++e) s = p[4 * e] <= x ? e : s;
+  const uint4 v = reinterpret_cast<const uint4*>(p)[s];
+  return slot_holds(r, x, v.y) ? w + ((uint64_t)v.z | ((uint64_t)v.w << 32)) : w;
 }
 
 }  // namespace fdy

@@ -268,23 +268,24 @@ int fdy_get_live(fdy_archive* a, void* stream, uint32_t template_graph, uint64_t
                  uint32_t* node_src, uint64_t node_cap, uint32_t* current_graph);
 
 /* Standalone relocation of packed u64 words already in device memory
- * (in and out may alias).  The plan holds the interval search structure:
- * about 16 root lines of 64 B per interval (2M intervals: about 2 GB of device
- * memory), built once for many relocations, against about 2 per interval for
- * the index beside a restored archive.  The table is checked on the host and
- * the index built on the current device (only the table is uploaded);
- * returns when it is built. */
+ * (in and out may alias).  The plan holds the table's interval search
+ * structure: up to 786,432 intervals, root entries of 16 B over lines of 64 B
+ * and the table itself (about 46 B per interval in all); past that, about 16
+ * root lines of 64 B per interval (2M intervals: about 2 GB of device
+ * memory).  The table is checked on the host and the index built on the
+ * current device (only the table is uploaded); returns when it is built. */
 int fdy_reloc_plan_create(const uint64_t* lo, const uint64_t* hi, const uint64_t* new_lo, uint64_t n,
                           uint32_t policy, fdy_reloc_plan** out);
 int fdy_reloc_plan_destroy(fdy_reloc_plan* p);
 int fdy_relocate_words(const fdy_reloc_plan* p, const uint64_t* d_in, uint64_t* d_out, uint64_t n_words,
                        void* stream);
-/* The plan's interval index: its 64-byte lines (the root lines first, then
- * the lines below them), copied to `lines` (room for cap of them) with their
- * count in *n_lines (lines may be null to ask for the count).  The index is
- * built on the device, one thread per root line.  No counterpart in the
- * reference; for inspecting a plan and checking the device build against
- * the host build of the same index. */
+/* The plan's table as an index of root lines: its 64-byte lines (the root
+ * lines first, then the lines below them), copied to `lines` (room for cap of
+ * them) with their count in *n_lines (lines may be null to ask for the count).
+ * The lines are built on the device, one thread per root line: with the plan
+ * where they are the index it searches, else when this is called.  No
+ * counterpart in the reference; for inspecting a plan's table and checking
+ * the device build against the host build of the same index. */
 int fdy_reloc_plan_lines(const fdy_reloc_plan* p, void* lines, uint64_t cap, uint64_t* n_lines);
 
 /* fdy_relocate_words without any device allocation.  No counterpart in the

@@ -1,0 +1,92 @@
+"""The two-level interval index at the edges of its parts: root entries that
+answer themselves, whose range holds one leaf (4 intervals), all seven (28) and one more (a tree of
+lines: 29, 60, 61, 900, 901), starts on the fences' unit and off it, one, two and
+256 entries more or less, a gap before every interval and none, both policies.
+On the CPU the host build and one lane's search, and on the GPU the device
+build and k_reloc's search by waves, against the oracle's binary search, bit for bit."""
+import json
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle
+from foundry_amd.restore import RelocPlan
+
+CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "_build", "reloc_roots_check")
+
+
+def _run_of(rng, at, count, unit, gap):
+    """count intervals of a few units each from `at`, abutting or with gaps."""
+    size = unit * rng.integers(1, 4, count).astype(np.uint64)
+    step = size + (unit * rng.integers(1, 3, count).astype(np.uint64) if gap else np.uint64(0))
+    lo = np.uint64(at) + np.cumsum(step, dtype=np.uint64) - step
+    return lo, lo + size
+
+
+def _table(kind, rng):
+    """Runs of the given lengths of small intervals, spread over a wide span."""
+    base = 0x7F0000000000
+    if kind == "one":
+        lo, hi = np.array([base], np.uint64), np.array([base + 12345], np.uint64)
+    elif kind in ("aligned", "unaligned", "bytes"):
+        unit = {"aligned": 256, "unaligned": 24, "bytes": 1}[kind]
+        parts = []
+        at = base
+        for rep in range(3):
+            for count in (1, 3, 4, 5, 27, 28, 29, 30, 60, 61, 900, 901):
+                parts.append(_run_of(rng, at, count, unit, gap=rep != 1))
+                at = int(parts[-1][1][-1]) + int(rng.integers(1, 64)) * (1 << 22)
+                at -= at % unit if kind == "aligned" else 0
+        lo, hi = (np.concatenate(x) for x in zip(*parts))
+    elif kind == "crowded":  # thousands under one entry beside one interval far away
+        lo, hi = _run_of(rng, base, 20000, 256, gap=False)
+        lo, hi = np.append(lo, np.uint64(base + (1 << 45))), np.append(hi, np.uint64(base + (1 << 45) + 4096))
+    else:  # n intervals of 100 kB or so; "wide": of up to 64 MB
+        n = int(kind.split("-")[0])
+        size = 256 * (1 + np.exp(rng.uniform(0, 12.5 if "wide" in kind else 7, n))).astype(np.uint64)
+        hi = np.uint64(base) + np.cumsum(size, dtype=np.uint64)
+        lo = hi - size
+    n = len(lo)
+    nlo = np.uint64(1 << 44) + rng.permutation(n).astype(np.uint64) * np.uint64(1 << 27)
+    edges = np.concatenate([lo - np.uint64(1), lo, lo + np.uint64(1), hi - np.uint64(1), hi, hi + np.uint64(1)])
+    inside = lo[0] + rng.integers(0, int(hi[-1] - lo[0]) + 2, 20001).astype(np.uint64)
+    return lo, hi, nlo, np.concatenate([edges, inside, np.array([0, (1 << 64) - 1], np.uint64)])
+
+
+KINDS = ["one", "2", "5", "aligned", "unaligned", "bytes", "crowded", "1021", "2048", "2049", "40000", "300-wide", "4096-wide"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_host_build_and_search(tmp_path, kind):
+    lo, hi, nlo, words = _table(kind, np.random.default_rng(KINDS.index(kind)))
+    t, w, o = (str(tmp_path / f) for f in ("t.bin", "w.bin", "o.bin"))
+    words.tofile(w)
+    for policy in (0, 1):
+        np.concatenate([np.array([len(lo), policy], np.uint64), lo, hi, nlo]).tofile(t)
+        p = subprocess.run([CHECK, t, w, o], capture_output=True, text=True, timeout=60)
+        assert p.returncode == 0, p.stderr
+        shape = json.loads(p.stdout)
+        assert kind not in ("aligned", "1021", "40000") or (shape["exact"] and shape["flat"] > 0), shape
+        assert kind != "bytes" or not shape["exact"], shape
+        assert kind == "one" or shape["direct"] > 0, shape
+        assert kind not in ("aligned", "unaligned", "bytes", "crowded") or shape["deep"] > 0, shape
+        np.testing.assert_array_equal(np.fromfile(o, np.uint64), oracle.relocate_words(words, lo, hi, nlo, policy))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+def test_device_build_and_search(cuda, kind):
+    lo, hi, nlo, words = _table(kind, np.random.default_rng(KINDS.index(kind)))
+    print(f"[case] two-level index: {kind}, {len(lo)} intervals, {len(words)} words", flush=True)
+    d_in = cuda.from_numpy(words.view(np.int64)).to("cuda")
+    for policy in (0, 1):
+        want = oracle.relocate_words(words, lo, hi, nlo, policy)
+        plan = RelocPlan(lo, hi, nlo, policy)
+        for start in (0, 1):  # 16-byte aligned words, and 8-byte aligned ones
+            d_out = cuda.zeros_like(d_in)
+            plan.relocate(d_in.data_ptr() + 8 * start, d_out.data_ptr() + 8 * start, len(words) - start)
+            cuda.cuda.synchronize()
+            np.testing.assert_array_equal(d_out.cpu().numpy().view(np.uint64)[start:], want[start:])
+        plan.close()
