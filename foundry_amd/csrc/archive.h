@@ -109,6 +109,12 @@ struct fdy_archive {
   uint32_t rec_shift = 0, cand_cap = 0, spill_cap = 0;
   bool live_ready = false;    // live images filled from this restore's R
   std::vector<uint64_t> h_live_base, h_r_base;  // h_r_base[g]: first word of R_g, packed to its words
+  // The sequence kernel's tables (SeqGraph per graph, records by tile), built
+  // when a sequence of switches first runs on a restore's results or on
+  // their serving layout.
+  fdy::DevBuf seq;
+  std::vector<uint32_t> h_seq_tiles;  // per graph: tiles of its template's words
+  bool seq_ready = false;
   bool use_explicit = false;
   bool restored = false;
   hipStream_t last_stream = nullptr;

@@ -106,6 +106,55 @@ static_assert(sizeof(SwitchBatch) <= 2048, "a switch batch travels as kernel arg
 uint32_t switch_blocks(const SwitchArgs& a);
 hipError_t launch_switch_many(const SwitchBatch& b, hipStream_t s);
 
+// A sequence of switches in one launch, cut by groups and by tiles of
+// kSeqWords template words: a workgroup makes all of its group's switches
+// within its tile (and its share of the group's nodes), so that no workgroup
+// waits for another.
+constexpr uint32_t kSeqWords = 1024;
+struct SeqGraph {
+  uint64_t rec;       // first override record
+  uint64_t num_rec;
+  uint64_t off;       // first entry of `offs`: per tile, the graph's records before it (and in all)
+  uint64_t live;      // (template) first word of the live image
+  uint64_t image;     // (template) first word of R
+  uint64_t node_base;
+  uint32_t num_nodes;
+  uint32_t words;     // words of the graph's template
+};
+// Tiles of a template of `words` words, at least one.
+__host__ __device__ inline uint32_t seq_tiles(uint32_t words) {
+  return words ? (uint32_t)(((uint64_t)words + kSeqWords - 1) / kSeqWords) : 1u;
+}
+// The tile table of every graph: offs[graphs[g].off + k] = the records of g
+// whose word lies before tile k, k = 0 .. seq_tiles.
+struct SeqIndexArgs {
+  const SeqGraph* graphs;
+  const fdy_override* ovr;
+  uint32_t* offs;
+  uint32_t num_graphs;
+};
+hipError_t launch_seq_index(const SeqIndexArgs& a, hipStream_t s);
+
+constexpr uint32_t kSeqGroups = 32;    // groups per launch
+constexpr uint32_t kSeqTargets = 704;  // list entries per launch: every group's current graph, then its targets
+struct SwitchSeq {
+  const SeqGraph* graphs;
+  const uint32_t* offs;
+  const fdy_override* ovr;
+  const uint64_t* image;
+  uint64_t* live;
+  const uint8_t* flags;    // node flags of all graphs
+  uint32_t* live_src;
+  uint32_t num_groups;
+  uint32_t pad_;
+  uint32_t tmpl[kSeqGroups];
+  uint32_t end[kSeqGroups];        // running workgroup counts (a group's tiles)
+  uint32_t first[kSeqGroups + 1];  // the group's entries of `target`
+  uint32_t target[kSeqTargets];
+};
+static_assert(sizeof(SwitchSeq) <= 4096, "a sequence travels as kernel arguments");
+hipError_t launch_switch_seq(const SwitchSeq& q, hipStream_t s);
+
 // Copy of the dirty nodes' live words (or of every node's) into the host
 // mirror of a group graph, with the dirty marks; clears the device marks.
 struct MirrorArgs {

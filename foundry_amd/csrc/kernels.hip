@@ -31,6 +31,8 @@
 //             gaps that compared words equal after relocation leave in a
 //             graph's override array closed.
 //   k_switch  override scatter for one graph switch.
+//   k_switch_seq  a sequence of switches, a workgroup per tile of a group's
+//             words (k_seq_index: every graph's records by tile).
 //   k_mirror  dirty nodes' live words -> a group graph's host mirror.
 //   k_fill    memset node of a restored graph, as a kernel node.
 //   k_reloc   streaming relocation of packed words.
@@ -2619,6 +2621,110 @@ __global__ __launch_bounds__(kSwitchThreads) void k_switch_many(SwitchBatch b) {
   switch_block(b.sw[k], blockIdx.x - first, b.end[k] - first, s_sample, s_seg);
 }
 
+// The tile tables (SeqIndexArgs), one workgroup per graph.
+__global__ __launch_bounds__(kSwitchThreads) void k_seq_index(SeqIndexArgs a) {
+  const uint32_t g = blockIdx.x;
+  const SeqGraph& G = a.graphs[g];
+  const fdy_override* rec = a.ovr + G.rec;
+  const uint64_t n = G.num_rec;
+  const uint32_t tiles = seq_tiles(G.words);
+  for (uint32_t k = threadIdx.x; k <= tiles; k += kSwitchThreads) {
+    uint64_t lo = 0, hi = k < tiles ? n : 0;  // the first record in tile k or past it
+    while (lo < hi) {
+      const uint64_t mid = (lo + hi) >> 1;
+      if (rec[mid].word < k * kSeqWords) lo = mid + 1;
+      else hi = mid;
+    }
+    a.offs[G.off + k] = (uint32_t)(k < tiles ? lo : n);
+  }
+}
+
+// A sequence of switches (SwitchSeq).  Per switch the workgroup (one wave)
+// stores the target's records of its tile and marks their words in a bitmap,
+// then stores the template's word (its tile of R lies in LDS) under every
+// record of the graph before that the bitmap does not hold.  The two sets are
+// disjoint, so only consecutive switches are ordered, by a barrier.  The next
+// switch's records are loaded ahead.
+//   Bound by the scattered stores, two per record and switch: 2000 switches
+// over 8 groups of 64 graphs x 5000 nodes (39,000 records each) took 3.04 ms
+// as a launch per 8 switches (k_switch_many: a gap and five rounds of loads in
+// a row each, one of them a search of the target's records), 1.37 ms with as
+// many workgroups as fit, whose live tiles (64 MB) the L2s cannot hold, so that
+// every store was written back as a part of a line, and 0.85 ms with eight per
+// CU (16 MB of live tiles), which the launch's LDS holds it to; 0.86 with 2048
+// words and two waves, 0.85 with 4096 and four, but a small group then has
+// too few workgroups.
+constexpr uint32_t kSeqThreads = 64;
+constexpr uint32_t kSeqLds = 20000;  // per workgroup: eight per CU of 160 KB
+constexpr uint32_t kSeqStaticLds = 8 * kSeqWords + 2 * kSeqWords / 8;
+static_assert(kSeqStaticLds < kSeqLds, "the tile and its bitmaps fit");
+
+__global__ __launch_bounds__(kSeqThreads) void k_switch_seq(SwitchSeq q) {
+  __shared__ uint64_t s_t[kSeqWords];
+  __shared__ uint32_t s_bits[2][kSeqWords / 32];
+  const uint32_t tid = threadIdx.x;
+  uint32_t j = 0;
+  while (j + 1 < q.num_groups && q.end[j] <= blockIdx.x) ++j;
+  const uint32_t tile = blockIdx.x - (j ? q.end[j - 1] : 0u), tmpl = q.tmpl[j];
+  const auto* T = readonly(q.graphs + tmpl);
+  const uint32_t w0 = tile * kSeqWords;
+  uint64_t* const live = q.live + T->live;
+  const uint64_t* const timg = q.image + T->image + w0;
+  const uint32_t words = T->words, tiles = seq_tiles(words);
+  // The tile's share of the group's nodes.
+  const uint32_t N = T->num_nodes;
+  const uint32_t n0 = (uint32_t)((uint64_t)N * tile / tiles), n1 = (uint32_t)((uint64_t)N * (tile + 1) / tiles);
+  uint32_t* const src = q.live_src + T->node_base;
+  // Graph g's records in this tile.
+  struct Range {
+    const uint4* rec;
+    uint32_t n;
+  };
+  auto range = [&](uint32_t g) -> Range {
+    const auto* G = readonly(q.graphs + g);
+    const auto* o = readonly(q.offs + G->off + tile);
+    const uint32_t r0 = o[0], r1 = o[1];
+    return {reinterpret_cast<const uint4*>(q.ovr + G->rec) + r0, r1 - r0};
+  };
+  static_assert(sizeof(fdy_override) == 16, "a record is one 16-byte load: {word, node, value}");
+  const uint32_t* list = q.target + q.first[j];
+  const uint32_t steps = q.first[j + 1] - q.first[j];  // the current graph, then its targets
+  Range cur = range(list[0]), next = range(list[1]);
+  uint32_t cw = tid < cur.n ? cur.rec[tid].x : 0u;  // this thread's first word of the current graph
+  uint4 rec = tid < next.n ? next.rec[tid] : uint4{0, 0, 0, 0};
+  for (uint32_t i = tid; i < min(kSeqWords, words - w0); i += kSeqThreads) s_t[i] = timg[i];
+  for (uint32_t i = tid; i < kSeqWords / 32; i += kSeqThreads) s_bits[0][i] = s_bits[1][i] = 0;
+  __syncthreads();
+  for (uint32_t s = 1; s < steps; ++s) {
+    const uint32_t g = list[s];
+    uint32_t* const bits = s_bits[s & 1];
+    auto put = [&](const uint4& r) {
+      live[r.x] = (uint64_t)r.z | ((uint64_t)r.w << 32);
+      atomicOr(bits + ((r.x - w0) >> 5), 1u << ((r.x - w0) & 31));
+    };
+    if (tid < next.n) put(rec);
+    for (uint32_t i = tid + kSeqThreads; i < next.n; i += kSeqThreads) put(next.rec[i]);
+    const Range after = range(list[min(s + 1, steps - 1)]);
+    lds_barrier();
+    auto back = [&](uint32_t w) {
+      const uint32_t l = w - w0;
+      if (!((bits[l >> 5] >> (l & 31)) & 1)) live[w] = s_t[l];
+    };
+    if (tid < cur.n) back(cw);
+    for (uint32_t i = tid + kSeqThreads; i < cur.n; i += kSeqThreads) back(cur.rec[i].x);
+    const uint8_t* fl = q.flags + readonly(q.graphs + g)->node_base;
+    for (uint32_t n = n0 + tid; n < n1; n += kSeqThreads)
+      src[n] = (fl[n] & (FDY_NODE_LAYOUT | FDY_NODE_DESC)) ? g : tmpl;
+    for (uint32_t i = tid; i < kSeqWords / 32; i += kSeqThreads) s_bits[(s & 1) ^ 1][i] = 0;
+    cw = rec.x;
+    cur = next;
+    next = after;
+    rec = tid < next.n ? next.rec[tid] : uint4{0, 0, 0, 0};
+    // The next switch's stores follow this one's; its bits follow the clearing.
+    __syncthreads();
+  }
+}
+
 // ---- interval index, built on the device ------------------------------
 
 // Exclusive prefix over the workgroup of one u64 per thread (kWaves waves);
@@ -3009,6 +3115,17 @@ uint32_t switch_blocks(const SwitchArgs& a) {
 hipError_t launch_switch_many(const SwitchBatch& b, hipStream_t s) {
   if (b.n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_switch_many, dim3(b.end[b.n - 1]), dim3(kSwitchThreads), 0, s, b);
+  return hipGetLastError();
+}
+
+hipError_t launch_seq_index(const SeqIndexArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_seq_index, dim3(a.num_graphs), dim3(kSwitchThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_switch_seq(const SwitchSeq& q, hipStream_t s) {
+  if (q.num_groups == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_switch_seq, dim3(q.end[q.num_groups - 1]), dim3(kSeqThreads), kSeqLds - kSeqStaticLds, s, q);
   return hipGetLastError();
 }
 

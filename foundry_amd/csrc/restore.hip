@@ -529,12 +529,13 @@ int compact_for_serving(fdy_archive* a, hipStream_t s) {
   a->aux.release();
   a->h_r_base = std::move(rbase);
   a->compact = true;
+  a->seq_ready = false;  // the records and images moved
   return FDY_OK;
 }
 
 uint64_t held_bytes(const fdy_archive* a) {
   const DevBuf* bufs[] = {&a->arena, &a->img, &a->image, &a->aux, &a->live, &a->ovr, &a->cand,
-                          &a->reloc.index};
+                          &a->reloc.index, &a->seq};
   uint64_t n = 0;
   for (const DevBuf* b : bufs) n += b->bytes;
   return n;
@@ -650,6 +651,43 @@ SwitchArgs switch_args(const fdy_archive* a, uint32_t g, uint8_t* dirty) {
   return switch_args(a, g, dirty, a->h_current[a->h_tmpl[g]]);
 }
 
+uint32_t* seq_offs(const fdy_archive* a) { return reinterpret_cast<uint32_t*>(a->seq.as<SeqGraph>() + a->G); }
+
+// The tables of the sequence kernel (every SeqGraph, then the tile tables);
+// synchronizes `s`.
+int build_seq_tables(fdy_archive* a, hipStream_t s) {
+  const uint32_t G = a->G;
+  std::vector<SeqGraph> sg(G);
+  a->h_seq_tiles.assign(G, 1);
+  uint64_t offs = 0;
+  for (uint32_t g = 0; g < G; ++g) {
+    const uint32_t t = a->h_tmpl[g];
+    a->h_seq_tiles[g] = seq_tiles(a->h_gwords[t]);
+    sg[g] = {ovr_base(a, g), a->h_ovr_off[g + 1] - a->h_ovr_off[g], offs, t == g ? live_base(a, g) : 0,
+             t == g ? r_base(a, g) : 0, a->graphs[g].node_base, a->graphs[g].num_nodes, a->h_gwords[t]};
+    offs += a->h_seq_tiles[g] + 1ull;
+  }
+  const uint64_t bytes = sizeof(SeqGraph) * G + 4 * offs;
+  if (a->seq.bytes < bytes) {
+    a->seq.release();
+    const int rc = dev_alloc(a->seq, bytes, "switch sequence tables");
+    if (rc) return rc;
+  }
+  FDY_HIP(hipMemcpyAsync(a->seq.p, sg.data(), sizeof(SeqGraph) * G, hipMemcpyHostToDevice, s));
+  FDY_HIP(launch_seq_index({a->seq.as<SeqGraph>(), a->ovr.as<fdy_override>(), seq_offs(a), G}, s));
+  FDY_HIP(hipStreamSynchronize(s));
+  a->seq_ready = true;
+  return FDY_OK;
+}
+
+// Whether `s` is being captured (nothing may be allocated or waited for).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 int enqueue_switch(fdy_archive* a, uint32_t g, hipStream_t s, uint8_t* dirty, bool set_device) {
   const uint32_t t = a->h_tmpl[g];
   if (a->h_current[t] == g) return FDY_OK;
@@ -746,6 +784,7 @@ int enqueue_restore(fdy_archive* a, hipStream_t s) {
   a->restored = true;
   a->cached = false;
   a->live_ready = false;
+  a->seq_ready = false;
   a->last_stream = s;
   return FDY_OK;
 }
@@ -1183,6 +1222,9 @@ int fdy_switch(fdy_archive* a, uint32_t g, void* stream) {
   return enqueue_switch(a, g, s, nullptr, true);
 }
 
+// Switches from which a sequence builds the sequence kernel's tables.
+constexpr uint64_t kSeqSwitches = 16;
+
 int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (!a) return err(FDY_E_INVALID, "null archive");
@@ -1225,6 +1267,70 @@ int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, voi
   bool layered = true;
   if (bound)
     for (uint64_t i = 0; i < n && layered; ++i) layered = !a->bound[a->h_tmpl[targets[i]]];
+  // A workgroup per tile of a group's words makes all of the group's switches
+  // there, so a sequence takes a launch per kSeqTargets switches (50 switches of
+  // one group of 8 graphs x 100 nodes: 34 us, by layers 140; of 4 groups of 16
+  // graphs x 400 nodes: 15 and 49).  Its tables cost a copy and a wait, about
+  // 50 us, once per restore: a few switches, and a stream under capture that
+  // finds none, take the layers below.
+  if (layered && !a->seq_ready && n >= kSeqSwitches && !capturing(s)) {
+    rc = build_seq_tables(a, s);
+    if (rc) return rc;
+  }
+  if (layered && a->seq_ready) {
+    SwitchSeq q{};
+    q.graphs = a->seq.as<SeqGraph>();
+    q.offs = seq_offs(a);
+    q.ovr = a->ovr.as<fdy_override>();
+    q.image = a->image.as<uint64_t>();
+    q.live = a->live.as<uint64_t>();
+    q.flags = a->nflags.as<uint8_t>();
+    q.live_src = a->live_src.as<uint32_t>();
+    std::vector<std::vector<uint32_t>> lists;  // per group of the launch: its current graph, then its targets
+    std::vector<uint32_t> slot(a->G, UINT32_MAX), cur = a->h_current;
+    uint32_t entries = 0;
+    auto launch = [&]() -> int {
+      q.num_groups = (uint32_t)lists.size();
+      uint32_t at = 0, blocks = 0;
+      for (uint32_t j = 0; j < q.num_groups; ++j) {
+        const uint32_t t = a->h_tmpl[lists[j][0]];
+        q.tmpl[j] = t;
+        blocks += a->h_seq_tiles[t];
+        q.end[j] = blocks;
+        q.first[j] = at;
+        std::copy(lists[j].begin(), lists[j].end(), q.target + at);
+        at += (uint32_t)lists[j].size();
+      }
+      q.first[q.num_groups] = at;
+      FDY_HIP(launch_switch_seq(q, s));
+      // A launch's switches are recorded as their groups' current graphs once
+      // it is enqueued.
+      for (const auto& l : lists) {
+        a->h_current[a->h_tmpl[l[0]]] = l.back();
+        slot[a->h_tmpl[l[0]]] = UINT32_MAX;
+      }
+      lists.clear();
+      entries = 0;
+      return FDY_OK;
+    };
+    for (uint64_t i = 0; i < n; ++i) {
+      const uint32_t g = targets[i], t = a->h_tmpl[g];
+      if (cur[t] == g) continue;
+      if (entries + 2 > kSeqTargets || (slot[t] == UINT32_MAX && lists.size() == kSeqGroups)) {
+        rc = launch();
+        if (rc) return rc;
+      }
+      if (slot[t] == UINT32_MAX) {
+        slot[t] = (uint32_t)lists.size();
+        lists.push_back({cur[t]});
+        ++entries;
+      }
+      lists[slot[t]].push_back(g);
+      ++entries;
+      cur[t] = g;
+    }
+    return lists.empty() ? FDY_OK : launch();
+  }
   if (layered) {
     std::vector<uint32_t> cur = a->h_current, depth(a->G, 0);
     std::vector<std::vector<std::pair<uint32_t, uint32_t>>> layers;  // {target, its group's graph before it}

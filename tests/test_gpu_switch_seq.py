@@ -1,0 +1,94 @@
+"""Switch sequences by tiles (k_switch_seq) at the edges of their splits:
+templates of less than a 1024-word tile, a tile more or less than full and
+many, words differing in none, some and nearly all of a tile (more records than
+a workgroup has threads), one group and more groups than one launch holds,
+more switches than one launch holds, layouts and descriptors that differ,
+no-op switches, and sequences again after single switches and after another
+restore.  Every template's live words, node sources and current graph equal
+the oracle's after each sequence."""
+import numpy as np
+import pytest
+
+from foundry_amd import synth
+from tests.parity import gpu_and_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _same_live(arch, ref, templates):
+    for t in templates:
+        w, src, cur = arch.live(t)
+        w2, src2, cur2 = ref.live(t)
+        assert cur == cur2, (t, cur, cur2)
+        assert np.array_equal(w, w2), f"template {t}: {np.flatnonzero(w != w2)[:8]}"
+        assert np.array_equal(src, src2), f"template {t}: node sources"
+
+
+@pytest.mark.parametrize("graphs,groups,nodes,blob,diff,layout,steps", [
+    (6, 1, 1, 64, 0.5, 0, 40),           # a few words
+    (6, 2, 16, 512, 0.05, 0, 40),        # 1024 words a graph or a little less
+    (6, 2, 17, 512, 0.05, 0, 40),        # and a little more
+    (12, 3, 300, 700, 0.0, 0, 100),      # no words differ
+    (12, 3, 300, 700, 0.03, 10, 300),    # layouts and descriptors
+    (8, 2, 60, 2048, 0.95, 0, 60),       # most words: more records than threads
+    (80, 40, 20, 256, 0.1, 5, 400),      # more groups than a launch holds
+    (10, 1, 50, 256, 0.1, 0, 1500),      # more switches than a launch holds
+])
+def test_sequences_against_the_oracle(cuda, graphs, groups, nodes, blob, diff, layout, steps):
+    print(f"[case] {steps} switches: {graphs} graphs x {nodes} nodes, {groups} groups, diff {diff}", flush=True)
+    s = synth.SynthArchive(synth.preset(
+        2, num_graphs=graphs, num_groups=groups, nodes_per_graph=nodes, min_blob_bytes=blob, max_blob_bytes=blob,
+        max_params=8, diff_lo=diff, diff_hi=diff, layout_var_pct=layout, num_intervals=64, seed=0x5E9 + steps + nodes))
+    arch, ref = gpu_and_oracle(s)
+    of = arch.groups()
+    templates = sorted(set(int(t) for t in of))
+    seq = [int(g) for g in synth.switch_sequence(steps, graphs, steps)]
+    seq[3:6] = [seq[2]] * 3  # no-op switches
+    for part in (seq[: steps // 2], seq[steps // 2:]):
+        arch.switch_sequence(part)
+        for g in part:
+            ref.switch(g)
+        _same_live(arch, ref, templates)
+    arch.switch(int(seq[0]))  # a single switch in between
+    ref.switch(int(seq[0]))
+    arch.switch_sequence(seq)
+    for g in seq:
+        ref.switch(g)
+    _same_live(arch, ref, templates)
+    arch.restore()  # the tables of the restore before are not this one's
+    arch.groups()
+    _, again = gpu_and_oracle(s)
+    arch.switch_sequence(seq)
+    for g in seq:
+        again.switch(g)
+    _same_live(arch, again, templates)
+    arch.close()
+
+
+def test_captured_sequence(cuda):
+    """A sequence under stream capture enqueues kernels only, with its tables
+    there (a longer sequence ran before) and without (it ran none): replays
+    scatter what the eager sequence does."""
+    s = synth.SynthArchive(synth.preset(2, num_graphs=8, num_groups=2, nodes_per_graph=40, num_intervals=64))
+    for tables in (False, True):
+        print(f"[case] captured switch sequence, tables {'built' if tables else 'missing'}", flush=True)
+        arch, ref = gpu_and_oracle(s)
+        templates = sorted(set(int(t) for t in arch.groups()))
+        if tables:
+            warm = [int(g) for g in synth.switch_sequence(1, 8, 40)]
+            arch.switch_sequence(warm)
+            for g in warm:
+                ref.switch(g)
+        seq = [int(g) for g in synth.switch_sequence(2, 8, 40)]
+        cuda.cuda.synchronize()
+        stream = cuda.cuda.Stream()
+        graph = cuda.cuda.CUDAGraph()
+        with cuda.cuda.graph(graph, stream=stream):
+            arch.switch_sequence(seq, stream)
+        for g in seq:
+            ref.switch(g)
+        for _ in range(3):  # the scatters leave the same live words from any state they left before
+            graph.replay()
+            cuda.cuda.synchronize()
+            _same_live(arch, ref, templates)
+        arch.close()
