@@ -197,6 +197,11 @@ struct IndexArgs {
   RelocRoot* root;      // two-level index
   RelocLine* line;
 };
+// The table's check (check_table's, of the intervals): workgroup b writes
+// {whether an interval is at fault, the OR of its starts' offsets} to
+// part[2 * b]; returns the workgroups in *blocks, at most kTableBlocks.
+constexpr uint32_t kTableBlocks = 256;
+hipError_t launch_table_check(const IndexArgs& a, uint64_t* part, uint32_t* blocks, hipStream_t s);
 hipError_t launch_index_count(const IndexArgs& a, hipStream_t s);
 hipError_t launch_index_place(const IndexArgs& a, hipStream_t s);
 hipError_t launch_roots_count(const IndexArgs& a, hipStream_t s);

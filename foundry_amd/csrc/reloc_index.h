@@ -44,6 +44,20 @@ struct IndexShape {
   uint64_t nb;
 };
 
+// What check_table asks of interval i (prev_hi: the hi before it, or lo).
+__host__ __device__ inline bool interval_ok(uint64_t lo, uint64_t hi, uint64_t prev_hi) {
+  return lo < hi && hi != UINT64_MAX && prev_hi <= lo;
+}
+
+// A table's arguments before its intervals are looked at.
+inline int check_table_args(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint64_t n, uint32_t policy,
+                            std::string* why) {
+  if (policy > FDY_RELOC_INCLUSIVE) *why = "unknown relocation policy";
+  else if (n && (!lo || !hi || !nlo)) *why = "null interval array";
+  else return FDY_OK;
+  return FDY_E_INVALID;
+}
+
 // Checks a table: sorted, non-overlapping, non-empty intervals below 2^64-1
 // spanning less than 2^54 bytes, fewer than 2^32 of them.  *off_bits gets
 // the OR of every lo - lo[0] (the starts' common alignment).
@@ -54,14 +68,13 @@ inline int check_table(const uint64_t* lo, const uint64_t* hi, const uint64_t* n
     return code;
   };
   *off_bits = 0;
-  if (policy > FDY_RELOC_INCLUSIVE) return err(FDY_E_INVALID, "unknown relocation policy");
+  if (const int rc = check_table_args(lo, hi, nlo, n, policy, why)) return rc;
   if (n == 0) return FDY_OK;
-  if (!lo || !hi || !nlo) return err(FDY_E_INVALID, "null interval array");
-  // One pass without branches (every LOAD pays for it); a table that fails
-  // is walked again for the first interval at fault.
-  uint64_t bits = 0, bad = (uint64_t)(lo[0] >= hi[0]) | (uint64_t)(hi[0] == UINT64_MAX);
+  // One pass without branches; a table that fails is walked again for the
+  // first interval at fault.
+  uint64_t bits = 0, bad = (uint64_t)!interval_ok(lo[0], hi[0], lo[0]);
   for (uint64_t i = 1; i < n; ++i) {
-    bad |= (uint64_t)(lo[i] >= hi[i]) | (uint64_t)(hi[i] == UINT64_MAX) | (uint64_t)(hi[i - 1] > lo[i]);
+    bad |= (uint64_t)!interval_ok(lo[i], hi[i], hi[i - 1]);
     bits |= lo[i] - lo[0];
   }
   for (uint64_t i = 0; bad && i < n; ++i) {

@@ -230,9 +230,10 @@ int build_reloc_index(const uint64_t* lo, const uint64_t* hi, const uint64_t* nl
 // 262,144 intervals fit three of the slots and are copied without a wait.
 constexpr uint64_t kStageSlot = 2ull << 20;
 constexpr uint32_t kStageSlots = 4;
+constexpr uint32_t kStageResults = 2 * kTableBlocks;
 struct TableStage {
   std::mutex mu;
-  uint8_t* host = nullptr;  // the slots, then 64 bytes for results, pinned
+  uint8_t* host = nullptr;  // the slots, then kStageResults words for results, pinned
   UploadLane lane;
   uint64_t* result() const { return reinterpret_cast<uint64_t*>(host + kStageSlots * kStageSlot); }
 };
@@ -241,7 +242,7 @@ TableStage g_stage;
 int stage_open() {
   if (!g_stage.host) {
     void* p = nullptr;
-    FDY_HIP(hipHostMalloc(&p, kStageSlots * kStageSlot + 64, hipHostMallocPortable));
+    FDY_HIP(hipHostMalloc(&p, kStageSlots * kStageSlot + 8 * kStageResults, hipHostMallocPortable));
     g_stage.host = static_cast<uint8_t*>(p);
   }
   int dev = 0;
@@ -272,11 +273,41 @@ int stage_table(uint8_t* dst, const uint64_t* const src[3], uint64_t n) {
   return FDY_OK;
 }
 
-// A count that the index kernels leave on the device, once they have run.
-int stage_result(const uint64_t* dev, uint64_t* out) {
-  FDY_HIP(hipMemcpyAsync(g_stage.result(), dev, 8, hipMemcpyDeviceToHost, g_stage.lane.st));
+// `words` words (at most kStageResults) that the index kernels leave on the
+// device, at g_stage.result() once the kernels have run.
+int stage_result(const uint64_t* dev, uint32_t words) {
+  FDY_HIP(hipMemcpyAsync(g_stage.result(), dev, 8ull * words, hipMemcpyDeviceToHost, g_stage.lane.st));
   FDY_HIP(hipStreamSynchronize(g_stage.lane.st));
-  *out = *g_stage.result();
+  return FDY_OK;
+}
+
+// check_table of the staged table at ia.lo (its arguments checked), by a
+// kernel.  A table at fault is walked on the host for its first fault.
+int check_staged(const IndexArgs& ia, const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint32_t policy,
+                 uint64_t* off_bits, std::string* why) {
+  DevBuf part;
+  int rc = dev_alloc(part, 8 * kStageResults, "interval table check");
+  if (rc) {
+    *why = g_err;
+    return rc;
+  }
+  uint32_t blocks = 0;
+  hipError_t e = launch_table_check(ia, part.as<uint64_t>(), &blocks, g_stage.lane.st);
+  if (e == hipSuccess && stage_result(part.as<uint64_t>(), 2 * blocks) != FDY_OK) {
+    *why = g_err;
+    return FDY_E_HIP;
+  }
+  if (e != hipSuccess) {
+    *why = std::string("the interval table's check failed: ") + hipGetErrorString(e);
+    return FDY_E_HIP;
+  }
+  uint64_t bad = 0;
+  *off_bits = 0;
+  for (uint32_t b = 0; b < blocks; ++b) {
+    bad |= g_stage.result()[2 * b];
+    *off_bits |= g_stage.result()[2 * b + 1];
+  }
+  if (bad || ia.n > 0xFFFFFFF0ull || (hi[ia.n - 1] - lo[0]) >> 54) return check_table(lo, hi, nlo, ia.n, policy, off_bits, why);
   return FDY_OK;
 }
 
@@ -296,8 +327,9 @@ int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interv
   ia.block_sum = sums.as<uint64_t>();
   ia.total = sums.as<uint64_t>() + nblocks;
   FDY_HIP(launch_index_count(ia, g_stage.lane.st));
-  rc = stage_result(ia.total, total);
+  rc = stage_result(ia.total, 1);
   if (rc) return rc;
+  *total = *g_stage.result();
   if (*total > kMaxIndexLines) return err(FDY_E_INVALID, "interval index too large");
   if (!out) return FDY_OK;
   rc = dev_alloc(*out, *total * sizeof(RelocLine), "interval index lines");
@@ -324,9 +356,9 @@ int place_roots(IndexArgs ia, const RootShape& sh, DevBuf* out, RelocDev* dev) {
   ia.total = work.as<uint64_t>() + nblocks;
   ia.ends = reinterpret_cast<uint32_t*>(work.as<uint64_t>() + nblocks + 1);
   FDY_HIP(launch_roots_count(ia, g_stage.lane.st));
-  uint64_t total = 0;
-  rc = stage_result(ia.total, &total);
+  rc = stage_result(ia.total, 1);
   if (rc) return rc;
+  const uint64_t total = *g_stage.result();
   if (total > kRootDirect) return err(FDY_E_INVALID, "interval index too large");
   const uint64_t root_bytes = (sh.nb * sizeof(RelocRoot) + 255) / 256 * 256;
   rc = dev_alloc(*out, root_bytes + total * sizeof(RelocLine), "interval index");
@@ -347,8 +379,13 @@ int place_roots(IndexArgs ia, const RootShape& sh, DevBuf* out, RelocDev* dev) {
 // intervals, 280 and 264 us at a million, 202 and 246 us at 400,000.
 constexpr uint64_t kRootedIntervals = 3ull << 18;
 
-// The index of a table checked and shaped on the host, built on the device
-// (only the table travels over PCIe).  A table is refused when its index of
+// Tables up to this are checked on the host (0.7 ns an interval) before
+// anything else; larger ones by a kernel once they are on the device, whose
+// result costs a wait of about 20 us.
+constexpr uint64_t kHostCheck = 32768;
+
+// A table's index, shaped on the host and built on the device (only the table
+// travels over PCIe).  A table is refused when its index of
 // `root_lines_per_interval` root lines has more than 32 bits can name.
 // plan: the device copy of the table stays (at out->table) for
 // fdy_reloc_plan_lines, unless the plan's own index is those lines.  Synchronizes.
@@ -358,29 +395,38 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
   out->index.release();
   out->table.release();
   std::string why;
-  uint64_t off_bits;
-  int rc = check_table(lo, hi, nlo, n, policy, &off_bits, &why);
+  uint64_t off_bits = 0;
+  int rc = n <= kHostCheck ? check_table(lo, hi, nlo, n, policy, &off_bits, &why)
+                           : check_table_args(lo, hi, nlo, n, policy, &why);
   if (rc) return err(rc, why);
   out->dev.policy = policy;
   if (n == 0) return FDY_OK;
-  const uint64_t span = hi[n - 1] - lo[0];
-  if (line_shape(span, n, root_lines_per_interval).nb > kMaxIndexLines)
-    return err(FDY_E_INVALID, "interval index too large");
   RelocDev d = out->dev;
   if (n > 1 || plan) {
     DevBuf table;
     rc = dev_alloc(table, 24 * n, "interval table");
-    if (rc) return rc;
-    std::lock_guard<std::mutex> stage(g_stage.mu);
-    rc = stage_open();
+    std::unique_lock<std::mutex> stage(g_stage.mu);
+    if (!rc) rc = stage_open();
     const uint64_t* const arrays[3] = {lo, hi, nlo};
     if (!rc) rc = stage_table(table.as<uint8_t>(), arrays, n);
-    if (rc) return rc;
+    if (rc) {
+      // No device for the table's check: the host's, so that a table at fault
+      // is reported as such all the same.
+      const std::string device_why = g_err;
+      if (n > kHostCheck)
+        if (const int bad = check_table(lo, hi, nlo, n, policy, &off_bits, &why)) return err(bad, why);
+      return err(rc, device_why);
+    }
     IndexArgs ia{};
     ia.lo = table.as<uint64_t>();
     ia.hi = ia.lo + n;
     ia.nlo = ia.lo + 2 * n;
     ia.n = n;
+    if (n > kHostCheck) rc = check_staged(ia, lo, hi, nlo, policy, &off_bits, &why);
+    if (rc) return err(rc, why);
+    const uint64_t span = hi[n - 1] - lo[0];
+    if (line_shape(span, n, root_lines_per_interval).nb > kMaxIndexLines)
+      return err(FDY_E_INVALID, "interval index too large");
     if (n == 1) {  // one delta: no index
       FDY_HIP(hipStreamSynchronize(g_stage.lane.st));
     } else if (plan && n > kRootedIntervals) {
@@ -396,7 +442,7 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
   d.n = n;
   d.lo_min = lo[0];
   d.hi_max = hi[n - 1];
-  d.span = span + (policy ? 1 : 0);
+  d.span = hi[n - 1] - lo[0] + (policy ? 1 : 0);
   d.delta = nlo[0] - lo[0];
   out->dev = d;
   return FDY_OK;

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 import oracle
+from foundry_amd._lib import FoundryError
 from foundry_amd.restore import RelocPlan
 
 CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "_build", "reloc_roots_check")
@@ -90,3 +91,34 @@ def test_device_build_and_search(cuda, kind):
             cuda.cuda.synchronize()
             np.testing.assert_array_equal(d_out.cpu().numpy().view(np.uint64)[start:], want[start:])
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [32768, 32769, 70001])
+def test_tables_at_fault_are_refused_with_their_first_fault(cuda, n):
+    """Tables of 32768 intervals and fewer are checked on the host, larger
+    ones on the device: the same faults, each at the table's ends and between
+    two workgroups' shares, with the same message; the whole table passes."""
+    print(f"[case] refused tables of {n} intervals", flush=True)
+    lo = np.uint64(1 << 40) + np.uint64(4096) * np.arange(n, dtype=np.uint64)
+    hi = lo + np.uint64(4096)
+    RelocPlan(lo, hi, lo).close()
+    for at in (0, 1, 255, 256, n - 1):
+        h = hi.copy()
+        h[at] = lo[at]
+        with pytest.raises(FoundryError, match=f"interval {at} is empty"):
+            RelocPlan(lo, h, lo)
+        if at:
+            h = hi.copy()
+            h[at - 1] += np.uint64(1)
+            with pytest.raises(FoundryError, match=f"intervals {at - 1} and {at} overlap"):
+                RelocPlan(lo, h, lo)
+    h = hi.copy()
+    h[-1] = np.uint64((1 << 64) - 1)
+    with pytest.raises(FoundryError, match=f"interval {n - 1} ends at 2"):
+        RelocPlan(lo, h, lo)
+    h[-1] = lo[0] + np.uint64(1 << 54)
+    with pytest.raises(FoundryError, match="span more than 2"):
+        RelocPlan(lo, h, lo)
+    with pytest.raises(FoundryError, match="policy"):
+        RelocPlan(lo, hi, lo, 2)
