@@ -233,7 +233,7 @@ constexpr uint32_t kStageSlots = 4;
 constexpr uint32_t kStageResults = 2 * kTableBlocks;
 struct TableStage {
   std::mutex mu;
-  uint8_t* host = nullptr;  // the slots, then kStageResults words for results, pinned
+  uint8_t* host = nullptr;  // the slots, then kStageResults words for results
   UploadLane lane;
   uint64_t* result() const { return reinterpret_cast<uint64_t*>(host + kStageSlots * kStageSlot); }
 };
@@ -242,7 +242,12 @@ TableStage g_stage;
 int stage_open() {
   if (!g_stage.host) {
     void* p = nullptr;
-    FDY_HIP(hipHostMalloc(&p, kStageSlots * kStageSlot + 8 * kStageResults, hipHostMallocPortable));
+    const size_t bytes = kStageSlots * kStageSlot + 8 * kStageResults;
+    if (hipHostMalloc(&p, bytes, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      p = std::malloc(bytes);  // unpinned: copies that the runtime stages
+      if (!p) return err(FDY_E_NOMEM, "interval table staging of " + std::to_string(bytes) + " bytes");
+    }
     g_stage.host = static_cast<uint8_t*>(p);
   }
   int dev = 0;
