@@ -1726,8 +1726,8 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
 // quad are in flight.
 //   Bound by requests: 4 ps each over the GPU where they hit the L2s, 18 ps
 // where they miss them, whatever their size up to 128 B (250 and 55 G/s
-// measured over 4 MB and 200 MB).  So the index is small (about 25 bytes per
-// interval up to 64,000 of them) and one more, cached, read deep.  20.5 M
+// measured over 4 MB and 200 MB).  So the index is small (25 to 53 bytes per
+// interval) and one more, cached, read deep.  20.5 M
 // words with 25% pointers by 40,000 intervals: 97 us, where 16 root lines of
 // 64 B per interval (41 MB) read by one lane each took 136 us; eight lanes per
 // 128-byte line were slower than four per 64 bytes (an L2 hit delivers 10.5

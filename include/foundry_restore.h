@@ -270,7 +270,7 @@ int fdy_get_live(fdy_archive* a, void* stream, uint32_t template_graph, uint64_t
 /* Standalone relocation of packed u64 words already in device memory
  * (in and out may alias).  The plan holds the table's interval search
  * structure: up to 786,432 intervals, root entries of 16 B over lines of 64 B
- * and the table itself (about 46 B per interval in all); past that, about 16
+ * and the table itself (50 to 80 B per interval in all); past that, about 16
  * root lines of 64 B per interval (2M intervals: about 2 GB of device
  * memory).  The table is checked on the host and the index built on the
  * current device (only the table is uploaded); returns when it is built. */
