@@ -2751,7 +2751,7 @@ __device__ inline uint64_t index_block_scan(uint64_t v, uint64_t* s_part, uint64
 }
 
 // The check of a table's intervals (launch_table_check), bound by the 16 bytes
-// read per interval: 3 us at 200,000 intervals, where the host's pass over the
+// read per interval: 6 us at 200,000 intervals, where the host's pass over the
 // same arrays, out of its caches, took 137 us of the plan's 385.
 constexpr uint32_t kTableThreads = 256;
 __global__ __launch_bounds__(kTableThreads) void k_table_check(IndexArgs a, uint64_t* part) {
@@ -2844,7 +2844,7 @@ __global__ __launch_bounds__(kIndexThreads) void k_index_place(IndexArgs a) {
 // entry its interval range, kept for the place pass.  The place pass gives
 // every line a thread: the lines of a workgroup's entries are consecutive,
 // so it stores them as whole runs whatever the entries' sizes are.
-//   Bound by latency at 200,000 intervals (10 us count, 14 us place, 4 us the
+//   Bound by latency at 200,000 intervals (7 us count, 14 us place, 2 us the
 // scan between them, for 5 MB); one thread per root line searching the table
 // and writing its subtree, as the index of root lines is built, takes 180, 250
 // and 59 us there, for 156 MB.
