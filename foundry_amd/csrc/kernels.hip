@@ -1835,11 +1835,10 @@ __device__ __forceinline__ void wave_search(const RelocDev& R, uint64_t* sw, con
 
 // Template graphs: relocate their words into R and the live image.  The
 // template slots listed by the node pass are cut into units of kTUnit words
-// (kTWords per thread, so one search batch), spread over the grid.  Four
-// words per thread suit small graphs; where graphs average 256K words or
-// more, eight (half as many units, each workgroup working through fewer in
-// turn) measured 108 -> 97 us on the MoE-style archive, while four keep the
-// decode-style pass at 10.9 us (13.0 us with eight).
+// (kTWords per thread), spread over the grid.  Four words per thread suit
+// small graphs; where graphs average 256K words or more, eight (half as many
+// units, each workgroup working through fewer in turn) take the MoE-style
+// restore from 316 to 314 us, while four keep the decode-style pass at 6.8 us.
 constexpr uint32_t kTThreads = 256;
 constexpr uint32_t kTLines = 8;  // lines in flight per quad
 constexpr uint64_t kTWideSlotsPerGraph = 64;  // 64 slots of 4096 words: 256K words per graph
@@ -1861,8 +1860,8 @@ __global__ __launch_bounds__(kTThreads) void k_diff_t(RestoreArgs a) {
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const RelocDev& R = a.reloc;
   const uint32_t units = *readonly(a.tslot_count) * kTUnitsPerTile;
-  // The next unit's slot descriptor is loaded while this unit is worked on
-  // (with eight words per thread: MoE-style 105 -> 97 us).  The node pass
+  // The next unit's slot descriptor is loaded while this unit is worked on.
+  // The node pass
   // lists the template slots' descriptors themselves, so the first one is
   // a single load.
   SlotDesc next{};
