@@ -109,12 +109,16 @@ struct fdy_archive {
   uint32_t rec_shift = 0, cand_cap = 0, spill_cap = 0;
   bool live_ready = false;    // live images filled from this restore's R
   std::vector<uint64_t> h_live_base, h_r_base;  // h_r_base[g]: first word of R_g, packed to its words
-  // The sequence kernel's tables (SeqGraph per graph, records by tile), built
-  // when a sequence of switches first runs on a restore's results or on
-  // their serving layout.
-  fdy::DevBuf seq;
+  // The sequence kernel's tables (SeqGraph per graph, records by tile): their
+  // room is the end of `live`, from byte seq_at (0: no room), and they are
+  // built, in stream order, when a sequence of switches first runs on a
+  // restore's results or on their serving layout.  seq_done is recorded behind
+  // the build, for sequences on other streams; seq_settled: it has been seen
+  // to have passed.
+  uint64_t seq_at = 0;
   std::vector<uint32_t> h_seq_tiles;  // per graph: tiles of its template's words
-  bool seq_ready = false;
+  bool seq_ready = false, seq_settled = false;
+  hipEvent_t seq_done = nullptr;
   bool use_explicit = false;
   bool restored = false;
   hipStream_t last_stream = nullptr;
@@ -140,6 +144,7 @@ struct fdy_archive {
   ~fdy_archive() {
     for (hipEvent_t& e : ev)
       if (e) (void)hipEventDestroy(e);
+    if (seq_done) (void)hipEventDestroy(seq_done);
   }
 };
 

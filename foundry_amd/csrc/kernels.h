@@ -125,14 +125,20 @@ struct SeqGraph {
 __host__ __device__ inline uint32_t seq_tiles(uint32_t words) {
   return words ? (uint32_t)(((uint64_t)words + kSeqWords - 1) / kSeqWords) : 1u;
 }
-// The tile table of every graph: offs[graphs[g].off + k] = the records of g
-// whose word lies before tile k, k = 0 .. seq_tiles.
+// The tables of graphs first .. first + num_graphs - 1, whose entries travel
+// as kernel arguments (nothing is staged, so nothing waits): graphs[first + i]
+// = g[i], and offs[g.off + k] = the records of g whose word lies before tile
+// k, k = 0 .. seq_tiles.
+constexpr uint32_t kSeqIndexGraphs = 64;
 struct SeqIndexArgs {
-  const SeqGraph* graphs;
+  SeqGraph* graphs;
   const fdy_override* ovr;
   uint32_t* offs;
+  uint32_t first;
   uint32_t num_graphs;
+  SeqGraph g[kSeqIndexGraphs];
 };
+static_assert(sizeof(SeqIndexArgs) <= 4096, "graph entries travel as kernel arguments");
 hipError_t launch_seq_index(const SeqIndexArgs& a, hipStream_t s);
 
 constexpr uint32_t kSeqGroups = 32;    // groups per launch

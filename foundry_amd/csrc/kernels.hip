@@ -2623,10 +2623,10 @@ __global__ __launch_bounds__(kSwitchThreads) void k_switch_many(SwitchBatch b) {
   switch_block(b.sw[k], blockIdx.x - first, b.end[k] - first, s_sample, s_seg);
 }
 
-// The tile tables (SeqIndexArgs), one workgroup per graph.
+// The tables of SeqIndexArgs, one workgroup per graph.
 __global__ __launch_bounds__(kSwitchThreads) void k_seq_index(SeqIndexArgs a) {
-  const uint32_t g = blockIdx.x;
-  const SeqGraph& G = a.graphs[g];
+  const SeqGraph& G = a.g[blockIdx.x];
+  if (threadIdx.x == 0) a.graphs[a.first + blockIdx.x] = G;
   const fdy_override* rec = a.ovr + G.rec;
   const uint64_t n = G.num_rec;
   const uint32_t tiles = seq_tiles(G.words);
@@ -3149,6 +3149,7 @@ hipError_t launch_switch_many(const SwitchBatch& b, hipStream_t s) {
 }
 
 hipError_t launch_seq_index(const SeqIndexArgs& a, hipStream_t s) {
+  if (a.num_graphs == 0) return hipSuccess;
   hipLaunchKernelGGL(k_seq_index, dim3(a.num_graphs), dim3(kSwitchThreads), 0, s, a);
   return hipGetLastError();
 }

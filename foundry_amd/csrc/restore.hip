@@ -613,6 +613,18 @@ int alloc_restore_buffers(fdy_archive* a) {
   return rc;
 }
 
+// Every graph's tiles (of its template's words); the bytes of the sequence
+// kernel's tables.
+uint64_t seq_layout(fdy_archive* a) {
+  uint64_t bytes = 0;
+  a->h_seq_tiles.resize(a->G);
+  for (uint32_t g = 0; g < a->G; ++g) {
+    a->h_seq_tiles[g] = seq_tiles(a->h_gwords[a->h_tmpl[g]]);
+    bytes += sizeof(SeqGraph) + 4 * (a->h_seq_tiles[g] + 1ull);
+  }
+  return bytes;
+}
+
 // The templates' live images, filled from R (after a restore, once its
 // results are settled).
 int fill_live(fdy_archive* a, hipStream_t s) {
@@ -625,11 +637,29 @@ int fill_live(fdy_archive* a, hipStream_t s) {
       live_words += a->graphs[g].word_cap;
     }
   const uint64_t bytes = 8 * std::max<uint64_t>(1, live_words);
-  if (a->live.bytes != bytes) {
+  // Room behind them for the sequence kernel's tables, so that a sequence of
+  // switches allocates nothing.  They take 56 B per graph and 4 B per 1024
+  // words of its template; where templates are so much longer than their
+  // members that this is over 1 MB and 1/64 of the param images, or memory is
+  // short, there is no room, and sequences run in layers.
+  uint64_t seq = seq_layout(a), words = 0;
+  for (uint32_t g = 0; g < G; ++g) words += a->h_gwords[g];
+  if (seq > (1ull << 20) + words / 8 ||
+      (!a->seq_done && hipEventCreateWithFlags(&a->seq_done, hipEventDisableTiming) != hipSuccess)) {
+    (void)hipGetLastError();
+    seq = 0;
+  }
+  if (a->live.bytes != bytes + seq) {
     a->live.release();
-    int rc = dev_alloc(a->live, bytes, "template live images");
+    int rc = dev_alloc(a->live, bytes + seq, "template live images");
+    if (rc && seq) {
+      (void)hipGetLastError();
+      seq = 0;
+      rc = dev_alloc(a->live, bytes, "template live images");
+    }
     if (rc) return rc;
   }
+  a->seq_at = seq ? bytes : 0;
   for (uint32_t g = 0; g < G; ++g)
     if (a->h_tmpl[g] == g && a->h_gwords[g])
       FDY_HIP(hipMemcpyAsync(a->live.as<uint64_t>() + lbase[g], a->image.as<uint64_t>() + r_base(a, g),
@@ -678,7 +708,7 @@ int compact_for_serving(fdy_archive* a, hipStream_t s) {
 
 uint64_t held_bytes(const fdy_archive* a) {
   const DevBuf* bufs[] = {&a->arena, &a->img, &a->image, &a->aux, &a->live, &a->ovr, &a->cand,
-                          &a->reloc.index, &a->seq};
+                          &a->reloc.index};
   uint64_t n = 0;
   for (const DevBuf* b : bufs) n += b->bytes;
   return n;
@@ -794,41 +824,58 @@ SwitchArgs switch_args(const fdy_archive* a, uint32_t g, uint8_t* dirty) {
   return switch_args(a, g, dirty, a->h_current[a->h_tmpl[g]]);
 }
 
-uint32_t* seq_offs(const fdy_archive* a) { return reinterpret_cast<uint32_t*>(a->seq.as<SeqGraph>() + a->G); }
+SeqGraph* seq_graphs(const fdy_archive* a) {
+  return reinterpret_cast<SeqGraph*>(a->live.as<uint8_t>() + a->seq_at);
+}
+uint32_t* seq_offs(const fdy_archive* a) { return reinterpret_cast<uint32_t*>(seq_graphs(a) + a->G); }
 
-// The tables of the sequence kernel (every SeqGraph, then the tile tables);
-// synchronizes `s`.
+// Enqueues the build of the sequence kernel's tables on `s`.
 int build_seq_tables(fdy_archive* a, hipStream_t s) {
-  const uint32_t G = a->G;
-  std::vector<SeqGraph> sg(G);
-  a->h_seq_tiles.assign(G, 1);
+  SeqIndexArgs x{};
+  x.graphs = seq_graphs(a);
+  x.ovr = a->ovr.as<fdy_override>();
+  x.offs = seq_offs(a);
   uint64_t offs = 0;
-  for (uint32_t g = 0; g < G; ++g) {
+  for (uint32_t g = 0; g < a->G; ++g) {
     const uint32_t t = a->h_tmpl[g];
-    a->h_seq_tiles[g] = seq_tiles(a->h_gwords[t]);
-    sg[g] = {ovr_base(a, g), a->h_ovr_off[g + 1] - a->h_ovr_off[g], offs, t == g ? live_base(a, g) : 0,
-             t == g ? r_base(a, g) : 0, a->graphs[g].node_base, a->graphs[g].num_nodes, a->h_gwords[t]};
+    x.g[x.num_graphs++] = {ovr_base(a, g), a->h_ovr_off[g + 1] - a->h_ovr_off[g], offs, t == g ? live_base(a, g) : 0,
+                           t == g ? r_base(a, g) : 0, a->graphs[g].node_base, a->graphs[g].num_nodes, a->h_gwords[t]};
     offs += a->h_seq_tiles[g] + 1ull;
+    if (x.num_graphs == kSeqIndexGraphs || g + 1 == a->G) {
+      FDY_HIP(launch_seq_index(x, s));
+      x.first += x.num_graphs;
+      x.num_graphs = 0;
+    }
   }
-  const uint64_t bytes = sizeof(SeqGraph) * G + 4 * offs;
-  if (a->seq.bytes < bytes) {
-    a->seq.release();
-    const int rc = dev_alloc(a->seq, bytes, "switch sequence tables");
-    if (rc) return rc;
-  }
-  FDY_HIP(hipMemcpyAsync(a->seq.p, sg.data(), sizeof(SeqGraph) * G, hipMemcpyHostToDevice, s));
-  FDY_HIP(launch_seq_index({a->seq.as<SeqGraph>(), a->ovr.as<fdy_override>(), seq_offs(a), G}, s));
-  FDY_HIP(hipStreamSynchronize(s));
+  FDY_HIP(hipEventRecord(a->seq_done, s));
   a->seq_ready = true;
+  a->seq_settled = false;
   return FDY_OK;
 }
 
-// Whether `s` is being captured (nothing may be allocated or waited for).
+// Whether `s` is being captured (nothing may be waited for).
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
   (void)hipGetLastError();
   return true;
+}
+
+// Orders `s` behind the build of the tables, which may be under way on another
+// stream.  False where that cannot be done: a capture does not wait for work
+// outside it.
+bool follow_seq_tables(fdy_archive* a, hipStream_t s) {
+  if (a->seq_settled) return true;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // asking for an event's state disturbs no capture
+  const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  a->seq_settled = hipEventQuery(a->seq_done) == hipSuccess;
+  if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (a->seq_settled) return true;
+  (void)hipGetLastError();  // not ready
+  if (capturing(s)) return false;
+  if (hipStreamWaitEvent(s, a->seq_done, 0) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
 }
 
 int enqueue_switch(fdy_archive* a, uint32_t g, hipStream_t s, uint8_t* dirty, bool set_device) {
@@ -1413,16 +1460,22 @@ int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, voi
   // A workgroup per tile of a group's words makes all of the group's switches
   // there, so a sequence takes a launch per kSeqTargets switches (50 switches of
   // one group of 8 graphs x 100 nodes: 34 us, by layers 140; of 4 groups of 16
-  // graphs x 400 nodes: 15 and 49).  Its tables cost a copy and a wait, about
-  // 50 us, once per restore: a few switches, and a stream under capture that
-  // finds none, take the layers below.
-  if (layered && !a->seq_ready && n >= kSeqSwitches && !capturing(s)) {
-    rc = build_seq_tables(a, s);
-    if (rc) return rc;
+  // graphs x 400 nodes: 15 and 49).  Its tables cost a launch per
+  // kSeqIndexGraphs graphs once per restore: a few switches, and a stream under
+  // capture that finds none, take the layers below.
+  bool tiles = false;
+  if (layered && a->seq_at) {
+    if (a->seq_ready) {
+      tiles = follow_seq_tables(a, s);
+    } else if (n >= kSeqSwitches && !capturing(s)) {
+      rc = build_seq_tables(a, s);
+      if (rc) return rc;
+      tiles = true;
+    }
   }
-  if (layered && a->seq_ready) {
+  if (tiles) {
     SwitchSeq q{};
-    q.graphs = a->seq.as<SeqGraph>();
+    q.graphs = seq_graphs(a);
     q.offs = seq_offs(a);
     q.ovr = a->ovr.as<fdy_override>();
     q.image = a->image.as<uint64_t>();

@@ -253,7 +253,12 @@ int fdy_switch(fdy_archive* a, uint32_t graph, void* stream);
  * measuring sustained switches).  Every group goes through its own switches
  * in sequence order; switches of different groups, which touch disjoint
  * state, share launches (unless a group graph holds one of the groups:
- * then the sequence's order is kept throughout).  Every target, and every
+ * then the sequence's order is kept throughout).  Like fdy_switch it waits
+ * only for a restore whose results no call has read yet; it then enqueues
+ * kernels and events and allocates nothing, so `stream` may be one under
+ * capture (such a capture holds until the next restore) and another thread
+ * may be capturing meanwhile (with a group graph's groups among the targets,
+ * their execs are updated as fdy_switch does).  Every target, and every
  * switch's launch size, is checked before any switch is enqueued: an
  * invalid target or a switch too large for one launch enqueues nothing.  A
  * HIP failure while enqueueing (or in a bound group graph's exec update)

@@ -6,6 +6,8 @@ more switches than one launch holds, layouts and descriptors that differ,
 no-op switches, and sequences again after single switches and after another
 restore.  Every template's live words, node sources and current graph equal
 the oracle's after each sequence."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -92,3 +94,72 @@ def test_captured_sequence(cuda):
             cuda.cuda.synchronize()
             _same_live(arch, ref, templates)
         arch.close()
+
+
+def _restored():
+    s = synth.SynthArchive(synth.preset(2, num_graphs=12, num_groups=2, nodes_per_graph=60, num_intervals=64))
+    arch, ref = gpu_and_oracle(s)
+    templates = sorted(set(int(t) for t in arch.groups()))  # the restore's results are read here
+    return arch, ref, templates
+
+
+def test_first_sequence_waits_for_nothing(cuda):
+    """The first sequence after a restore, which builds the tables, returns
+    while the work queued on its stream before it is still running; a sequence
+    on another stream, of the other group, comes behind the tables."""
+    print("[case] first switch sequence behind a running kernel, and one on another stream", flush=True)
+    arch, ref, templates = _restored()
+    of = arch.groups()
+    own = [[int(g) for g in np.flatnonzero(of == t)] for t in templates]
+    first, second = (own[k][1:] * 8 for k in range(2))
+    a, b = cuda.cuda.Stream(), cuda.cuda.Stream()
+    with cuda.cuda.stream(a):
+        cuda.cuda._sleep(100_000_000)
+        slept = cuda.cuda.Event()
+        slept.record(a)
+    arch.switch_sequence(first, a)
+    running = not slept.query()
+    arch.switch_sequence(second, b)
+    running_after = not slept.query()
+    cuda.cuda.synchronize()
+    assert running and running_after
+    for g in first + second:
+        ref.switch(g)
+    _same_live(arch, ref, templates)
+    arch.close()
+
+
+def test_first_sequence_beside_a_capture_on_another_thread(cuda):
+    """A thread's sequence, the first after a restore, on its own stream while
+    another thread captures in the global mode: it runs, and the capture stays
+    whole."""
+    print("[case] first switch sequence while another thread captures", flush=True)
+    arch, ref, templates = _restored()
+    seq = [int(g) for g in synth.switch_sequence(3, 12, 40)]
+    own, cap, graph = cuda.cuda.Stream(), cuda.cuda.Stream(), cuda.cuda.CUDAGraph()
+    x = cuda.zeros(1000, device="cuda")
+    failed = []
+
+    def switches():
+        try:
+            arch.switch_sequence(seq, own)
+        except Exception as e:  # reported below, once the capture has ended
+            failed.append(e)
+
+    cuda.cuda.synchronize()
+    with cuda.cuda.graph(graph, stream=cap, capture_error_mode="global"):
+        x.add_(1)
+        t = threading.Thread(target=switches)
+        t.start()
+        t.join()
+        x.add_(1)
+    assert not failed, failed
+    own.synchronize()
+    for g in seq:
+        ref.switch(g)
+    _same_live(arch, ref, templates)
+    for k in (1, 2, 3):
+        graph.replay()
+        cuda.cuda.synchronize()
+        assert x.eq(2.0 * k).all()
+    arch.close()
