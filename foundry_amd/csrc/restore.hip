@@ -1415,6 +1415,31 @@ int fdy_switch(fdy_archive* a, uint32_t g, void* stream) {
 // Switches from which a sequence builds the sequence kernel's tables.
 constexpr uint64_t kSeqSwitches = 16;
 
+// What a sequence of switches takes by layers and by tiles.
+struct SeqShape {
+  uint64_t layers = 0, launches = 0;  // by layers: layers, and launches of up to kSwitchBatch switches
+  uint64_t records = 0;               // of all targets
+  uint64_t tiles = 0;                 // of all groups involved
+};
+
+// Whether a sequence with its tables built goes by tiles.  As long as the
+// groups' tiles are on the GPU together (2048: eight per CU) they win from the
+// second layer on: 50,000 to 1 M words a group, up to 34,000 records a switch,
+// two layers 6.4 to 7.1 us against 8.3 to 9.9 by layers, eight 10 to 12 against
+// 26 to 40; one switch is one launch either way (alone 17.4 us by layers, 18.6
+// by tiles).  More tiles come in rounds, each staging its tiles of R first and
+// then paying every switch's steps again, where a launch of a layer takes 4.5
+// us and 40 ps a record.  4 groups of 990,000 words, 2600 records a switch:
+// six layers 26.6 us (tiles 27.9), eight 35.9 (32.2); of 34,000 records: two
+// 16.6 (21.4), four 33.0 (26.8).  8 such groups: sixteen 85 (83), thirty-two
+// 170 (125); of 34,000 records: two 30 (40), four 59 (50).
+bool by_tiles(const SeqShape& q) {
+  constexpr uint64_t kResident = 8 * 256;
+  if (q.tiles <= kResident) return q.layers >= 2;
+  const uint64_t rounds = (q.tiles + kResident - 1) / kResident;
+  return 4500 * q.launches + q.records / 25 > rounds * (11000 + 700 * q.layers);  // ns
+}
+
 int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (!a) return err(FDY_E_INVALID, "null archive");
@@ -1432,8 +1457,10 @@ int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, voi
   // point of the sequence: follow the sequence on a copy first, so that a
   // switch too large for one launch refuses the whole sequence before
   // anything is enqueued.
+  SeqShape shape;
   {
-    std::vector<uint32_t> cur = a->h_current;
+    std::vector<uint32_t> cur = a->h_current, depth(a->G, 0);
+    std::vector<uint64_t> in_layer;
     for (uint64_t i = 0; i < n; ++i) {
       const uint32_t g = targets[i], t = a->h_tmpl[g];
       if ((bound && a->bound[t]) || cur[t] == g) continue;
@@ -1441,7 +1468,14 @@ int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, voi
         return err(FDY_E_CAPACITY, "override sets too large for one switch launch (target " +
                                        std::to_string(g) + ")");
       cur[t] = g;
+      const uint32_t k = depth[t]++;
+      if (k == 0) shape.tiles += a->h_seq_tiles[t];
+      if (k == in_layer.size()) in_layer.push_back(0);
+      ++in_layer[k];
+      shape.records += a->h_ovr_off[g + 1] - a->h_ovr_off[g];
     }
+    shape.layers = in_layer.size();
+    for (const uint64_t m : in_layer) shape.launches += (m + kSwitchBatch - 1) / kSwitchBatch;
   }
   FDY_HIP(hipSetDevice(a->device));
   // Switches of different groups touch disjoint live images and node
@@ -1457,14 +1491,15 @@ int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, voi
   bool layered = true;
   if (bound)
     for (uint64_t i = 0; i < n && layered; ++i) layered = !a->bound[a->h_tmpl[targets[i]]];
-  // A workgroup per tile of a group's words makes all of the group's switches
-  // there, so a sequence takes a launch per kSeqTargets switches (50 switches of
-  // one group of 8 graphs x 100 nodes: 34 us, by layers 140; of 4 groups of 16
-  // graphs x 400 nodes: 15 and 49).  Its tables cost a launch per
-  // kSeqIndexGraphs graphs once per restore: a few switches, and a stream under
-  // capture that finds none, take the layers below.
+  // By tiles (by_tiles), a workgroup per tile of a group's words makes all of
+  // the group's switches there, so a sequence takes a launch per kSeqTargets
+  // switches (50 switches of one group of 8 graphs x 100 nodes: 34 us, by
+  // layers 140; of 4 groups of 16 graphs x 400 nodes: 15 and 49).  The tables
+  // cost a launch per kSeqIndexGraphs graphs once per restore: fewer than
+  // kSeqSwitches switches, and a stream under capture that finds none, take the
+  // layers below.
   bool tiles = false;
-  if (layered && a->seq_at) {
+  if (layered && a->seq_at && by_tiles(shape)) {
     if (a->seq_ready) {
       tiles = follow_seq_tables(a, s);
     } else if (n >= kSeqSwitches && !capturing(s)) {

@@ -163,3 +163,27 @@ def test_first_sequence_beside_a_capture_on_another_thread(cuda):
         cuda.cuda.synchronize()
         assert x.eq(2.0 * k).all()
     arch.close()
+
+
+@pytest.mark.parametrize("graphs,groups,nodes,blob", [
+    (8, 2, 40, 256),      # all tiles on the GPU together
+    (9, 3, 5000, 1600),   # 2930 tiles, two rounds of them: layers for short sequences
+])
+def test_short_sequences_with_tables(cuda, graphs, groups, nodes, blob):
+    """Sequences on either side of the rule that chooses layers or tiles, one
+    after another on an archive whose tables are built: each leaves the live
+    words that the oracle's switches leave, whichever kernel it took."""
+    print(f"[case] short sequences: {graphs} graphs x {nodes} nodes, {groups} groups", flush=True)
+    s = synth.SynthArchive(synth.preset(
+        2, num_graphs=graphs, num_groups=groups, nodes_per_graph=nodes, min_blob_bytes=blob, max_blob_bytes=blob,
+        max_params=8, diff_lo=0.03, diff_hi=0.03, num_intervals=64, seed=0x5E9A + nodes))
+    arch, ref = gpu_and_oracle(s)
+    of = arch.groups()
+    own = [[int(g) for g in np.flatnonzero(of == t)] for t in sorted(set(int(t) for t in of))]
+    for layers in (40, 1, 2, 3, 4, 12, 1, 16):
+        seq = [m[(k + layers) % len(m)] for k in range(layers) for m in own]
+        arch.switch_sequence(seq)
+        for g in seq:
+            ref.switch(g)
+        _same_live(arch, ref, [m[0] for m in own])
+    arch.close()
