@@ -390,6 +390,9 @@ __host__ __device__ inline RelocRoot root_entry(uint64_t s0, uint64_t i, uint64_
     return r;
   }
   const bool flat = root_flat(j - i + 1, exact);
+  uint32_t levels = 0;  // of fence lines: at most 8 below 2^32 intervals
+  if (!flat)
+    for (uint64_t w = kLeafIntervals; w < j - i + 1; w *= kLineKids) ++levels;
   r.line = (uint32_t)first | (flat ? 0u : kRootTree);
   for (uint32_t e = 0; e < kRootFences / 2; ++e) {
     uint32_t f[2];
@@ -399,6 +402,7 @@ __host__ __device__ inline RelocRoot root_entry(uint64_t s0, uint64_t i, uint64_
     }
     r.word[e] = f[0] | (f[1] << 16);
   }
+  if (!flat) r.word[kRootFences / 2 - 1] = 0xFFFFu | (0xFFFFu - kRootLevels + levels) << 16;
   return r;
 }
 

@@ -193,11 +193,13 @@ __host__ __device__ inline uint32_t* line_fences(RelocLine& L) { return reinterp
 // it).  Otherwise the leaf lines line .. line + 6 hold the range's intervals
 // (as many as it has fences, and one), child c starting at fence c - 1 (child
 // 0 at the entry's first address), or (kRootTree) the fence line at the top
-// of a tree whose descent goes on as above.  A fence is an offset inside the
+// of a tree whose descent goes on as above (the last fence is then 0xFFF0 plus
+// the fence lines that a descent meets).  A fence is an offset inside the
 // entry's range in units of 2^fence_shift, below 2^15 (unused: 0xFFFF).  Line
 // 0 moves nothing: a search through a direct entry ends there.
 constexpr uint32_t kRootFences = 6;
 constexpr uint32_t kRootFenceBits = 15;
+constexpr uint32_t kRootLevels = 15;
 constexpr uint32_t kRootTree = 0x80000000u;
 constexpr uint32_t kRootDirect = 0x40000000u;  // also the line count's limit
 struct RelocRoot {
@@ -357,13 +359,14 @@ __host__ __device__ __forceinline__ bool slot_holds(const RelocDev& r, uint32_t 
   return r.policy ? x + 1 <= end : x + 1 < end;
 }
 
-// The leaf under fence line `line` that holds offset *x of it; *x becomes the
-// offset inside the leaf.
-__host__ __device__ __forceinline__ uint32_t tree_leaf(const RelocDev& r, uint32_t line, uint32_t* x) {
-  for (;;) {
+// The leaf under root entry rt's tree (its top: fence line `line`) that holds
+// offset *x of the entry's range; *x becomes the offset inside the leaf.  The
+// entry says how many fence lines there are above it, so the leaf is not read
+// to find out.
+__host__ __device__ __forceinline__ uint32_t tree_leaf(const RelocDev& r, const uint4& rt, uint32_t line, uint32_t* x) {
+  for (uint32_t l = (rt.w >> 16) & kRootLevels; l; --l) {
     const uint4* p = reinterpret_cast<const uint4*>(r.line + line);
     const uint4 v[kLineSlots] = {p[0], p[1], p[2], p[3]};
-    if (!(v[0].x & kLineFence)) return line;
     const uint32_t f[kLineFences] = {v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w, v[2].x,
                                      v[2].y, v[2].z, v[2].w, v[3].x, v[3].y, v[3].z, v[3].w};
     uint32_t c = 0, at = 0;
@@ -376,6 +379,7 @@ __host__ __device__ __forceinline__ uint32_t tree_leaf(const RelocDev& r, uint32
     *x -= at;
     line = v[0].y + c;
   }
+  return line;
 }
 
 // One word through the two-level index, by one lane (the kernels' searches go
@@ -389,7 +393,7 @@ __host__ __device__ inline uint64_t reloc_word(const RelocDev& r, uint64_t w) {
   const uint4 rt = *reinterpret_cast<const uint4*>(r.root + b);
   if (rt.x & kRootDirect) return slot_holds(r, x, rt.y) ? w + ((uint64_t)rt.z | ((uint64_t)rt.w << 32)) : w;
   uint32_t line = root_child(rt, r.fence_shift, &x);
-  if (rt.x & kRootTree) line = tree_leaf(r, line, &x);
+  if (rt.x & kRootTree) line = tree_leaf(r, rt, line, &x);
   const uint32_t* p = reinterpret_cast<const uint32_t*>(r.line + line);
   uint32_t s = 0;
 #pragma unroll

@@ -122,3 +122,27 @@ def test_tables_at_fault_are_refused_with_their_first_fault(cuda, n):
         RelocPlan(lo, h, lo)
     with pytest.raises(FoundryError, match="policy"):
         RelocPlan(lo, hi, lo, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("intervals", [2, 64, 1000, 40000])
+def test_restore_by_a_crowded_table(cuda, intervals):
+    """An archive's allocations under one root entry (another one lies 2^45
+    bytes away), so that every search of the template and search passes descends
+    a tree, in batches of a few words and of many: the oracle's restore."""
+    from foundry_amd import synth
+    from foundry_amd.restore import Archive
+    from tests.parity import assert_restore_parity
+
+    print(f"[case] restore by a crowded table of {intervals} intervals", flush=True)
+    s = synth.SynthArchive(synth.preset(2, num_graphs=12, num_groups=3, nodes_per_graph=200, num_intervals=intervals,
+                                        diff_lo=0.1, diff_hi=0.1, pointer_frac=0.4, seed=0x5EEDC0 + intervals))
+    lo, hi, nlo = (np.asarray(a) for a in s.intervals())
+    far = np.uint64(int(lo[0]) + (1 << 45))
+    table = np.append(lo, far), np.append(hi, far + np.uint64(4096)), np.append(nlo, np.uint64(1 << 46))
+    for policy in (0, 1):
+        arch = Archive.from_synth(s)
+        arch.set_relocation(*table, policy=policy)
+        arch.restore()
+        assert_restore_parity(arch, oracle.Restore(s.images(), table, policy=policy, threads=4))
+        arch.close()
