@@ -317,10 +317,10 @@ int check_staged(const IndexArgs& ia, const uint64_t* lo, const uint64_t* hi, co
 }
 
 // The index of root lines of the table at ia.lo, ia.hi, ia.nlo (device
-// memory; a checked table): *total lines, at `out` unless out is null.  On the
-// open stage's stream; synchronizes it.
-int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interval, DevBuf* out, uint64_t* total,
-                     uint32_t* shift) {
+// memory; a checked table): *total lines, placed at `out` unless they are more
+// than `cap`.  On the open stage's stream; synchronizes it.
+int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interval, uint64_t cap, DevBuf* out,
+                     uint64_t* total, uint32_t* shift) {
   const IndexShape sh = line_shape(span, ia.n, root_lines_per_interval);
   *shift = sh.shift;
   const uint64_t nblocks = (sh.nb + kIndexThreads - 1) / kIndexThreads;
@@ -336,7 +336,7 @@ int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interv
   if (rc) return rc;
   *total = *g_stage.result();
   if (*total > kMaxIndexLines) return err(FDY_E_INVALID, "interval index too large");
-  if (!out) return FDY_OK;
+  if (*total > cap) return FDY_OK;
   rc = dev_alloc(*out, *total * sizeof(RelocLine), "interval index lines");
   if (rc) return rc;
   ia.line = out->as<RelocLine>();
@@ -436,7 +436,7 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
       FDY_HIP(hipStreamSynchronize(g_stage.lane.st));
     } else if (plan && n > kRootedIntervals) {
       uint64_t total = 0;
-      rc = place_root_lines(ia, span, root_lines_per_interval, &out->index, &total, &d.shift);
+      rc = place_root_lines(ia, span, root_lines_per_interval, kMaxIndexLines, &out->index, &total, &d.shift);
       d.line = out->index.as<RelocLine>();
     } else {
       rc = place_roots(ia, root_shape(lo, hi, n, off_bits), &out->index, &d);
@@ -1858,7 +1858,8 @@ int fdy_reloc_plan_lines(const fdy_reloc_plan* p, void* lines, uint64_t cap, uin
     uint32_t shift = 0;
     std::lock_guard<std::mutex> stage(g_stage.mu);
     int rc = stage_open();
-    if (!rc) rc = place_root_lines(ia, d.hi_max - d.lo_min, kPlanRootLinesPerInterval, lines ? &built : nullptr, &n, &shift);
+    if (!rc)
+      rc = place_root_lines(ia, d.hi_max - d.lo_min, kPlanRootLinesPerInterval, lines ? cap : 0, &built, &n, &shift);
     if (rc) return rc;
     line = built.p;
   }

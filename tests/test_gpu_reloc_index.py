@@ -9,6 +9,7 @@ random gaps with abutting intervals, the widest root lines over a sparse
 span, one interval, a table at the top of the address space, and the
 relocation-heavy workload's interval mix.  Each plan then relocates its
 table's edge words as the oracle does."""
+import ctypes as C
 import os
 import subprocess
 
@@ -18,13 +19,14 @@ import torch
 
 import oracle
 from foundry_amd import synth
-from foundry_amd._lib import RELOC_HALF_OPEN, RELOC_INCLUSIVE
+from foundry_amd._lib import RELOC_HALF_OPEN, RELOC_INCLUSIVE, check, restore_lib
 from foundry_amd.restore import RelocPlan
 
 pytestmark = pytest.mark.gpu
 
 CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "_build", "reloc_index_check")
 PLAN_ROOT_LINES_PER_INTERVAL = 16
+FDY_E_CAPACITY = -8
 
 
 def _host_lines(tmp_path, lo, hi, nlo, policy):
@@ -98,3 +100,20 @@ def test_relocation_heavy_interval_mix(tmp_path):
     s = synth.SynthArchive(synth.preset(4, num_words=1 << 10))
     lo, hi, nlo = s.intervals()
     _check(tmp_path, "relocation-heavy mix (2M intervals)", lo, hi, nlo)
+
+
+def test_lines_with_too_little_room():
+    """A plan's lines are counted before any are built: too small an output is
+    refused with their count, and written nothing to."""
+    lo = np.uint64(1 << 40) + np.uint64(4096) * np.arange(5000, dtype=np.uint64)
+    print(f"[case] plan lines with too little room: {len(lo)} intervals", flush=True)
+    plan = RelocPlan(lo, lo + np.uint64(4096), lo)
+    want = plan.lines()
+    n = C.c_uint64()
+    out = np.full((len(want), 8), 7, np.uint64)
+    for cap in (0, 1, len(want) - 1):
+        rc = restore_lib().fdy_reloc_plan_lines(plan._h, out.ctypes.data_as(C.c_void_p), cap, C.byref(n))
+        assert rc == FDY_E_CAPACITY and n.value == len(want) and (out == 7).all()
+    check(restore_lib().fdy_reloc_plan_lines(plan._h, out.ctypes.data_as(C.c_void_p), len(want), C.byref(n)))
+    np.testing.assert_array_equal(out, want)
+    plan.close()
