@@ -12,6 +12,7 @@
 #include <atomic>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -224,8 +225,9 @@ int build_reloc_index(const uint64_t* lo, const uint64_t* hi, const uint64_t* nl
 }
 
 // The upload of interval tables: pinned slots of their own (a program
-// that only builds plans need not hold the ring) and a lane that the index
-// kernels run on as well, so that nothing waits between the copy and them.
+// that only builds plans need not hold the ring) and, per device, a lane that
+// the index kernels run on as well, so that nothing waits between the copy and
+// them.
 // The lock holds from stage_open() until the index is built.  Tables of up to
 // 262,144 intervals fit three of the slots and are copied without a wait.
 constexpr uint64_t kStageSlot = 2ull << 20;
@@ -234,7 +236,8 @@ constexpr uint32_t kStageResults = 2 * kTableBlocks;
 struct TableStage {
   std::mutex mu;
   uint8_t* host = nullptr;  // the slots, then kStageResults words for results
-  UploadLane lane;
+  std::map<int, UploadLane> lanes;
+  UploadLane* lane = nullptr;  // the open stage's, or the last one's
   uint64_t* result() const { return reinterpret_cast<uint64_t*>(host + kStageSlots * kStageSlot); }
 };
 TableStage g_stage;
@@ -252,17 +255,20 @@ int stage_open() {
   }
   int dev = 0;
   FDY_HIP(hipGetDevice(&dev));
-  if (!g_stage.lane.open(dev)) {
+  UploadLane& lane = g_stage.lanes[dev];
+  if (!lane.open(dev)) {
     (void)hipGetLastError();
     return err(FDY_E_HIP, "cannot create an upload stream or event");
   }
-  FDY_HIP(hipStreamSynchronize(g_stage.lane.st));  // a call that failed part-way may have left copies
+  // A call that failed part-way may have left copies out of the slots.
+  if (g_stage.lane) FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
+  g_stage.lane = &lane;
   return FDY_OK;
 }
 
 // The three arrays of n words to `dst`, end to end, in stream order.
 int stage_table(uint8_t* dst, const uint64_t* const src[3], uint64_t n) {
-  const hipStream_t st = g_stage.lane.st;
+  const hipStream_t st = g_stage.lane->st;
   uint32_t k = 0;
   for (uint32_t a = 0; a < 3; ++a)
     for (uint64_t at = 0; at < 8 * n; at += kStageSlot, ++k) {
@@ -270,10 +276,10 @@ int stage_table(uint8_t* dst, const uint64_t* const src[3], uint64_t n) {
       uint8_t* slot = g_stage.host + (k % kStageSlots) * kStageSlot;
       // The slots are refilled in halves: an event per half.
       constexpr uint32_t kHalf = kStageSlots / 2;
-      if (k >= kStageSlots && k % kHalf == 0) FDY_HIP(hipEventSynchronize(g_stage.lane.ev[k / kHalf & 1]));
+      if (k >= kStageSlots && k % kHalf == 0) FDY_HIP(hipEventSynchronize(g_stage.lane->ev[k / kHalf & 1]));
       std::memcpy(slot, reinterpret_cast<const uint8_t*>(src[a]) + at, len);
       FDY_HIP(hipMemcpyAsync(dst + 8 * n * a + at, slot, len, hipMemcpyHostToDevice, st));
-      if (k % kHalf == kHalf - 1) FDY_HIP(hipEventRecord(g_stage.lane.ev[k / kHalf & 1], st));
+      if (k % kHalf == kHalf - 1) FDY_HIP(hipEventRecord(g_stage.lane->ev[k / kHalf & 1], st));
     }
   return FDY_OK;
 }
@@ -281,8 +287,8 @@ int stage_table(uint8_t* dst, const uint64_t* const src[3], uint64_t n) {
 // `words` words (at most kStageResults) that the index kernels leave on the
 // device, at g_stage.result() once the kernels have run.
 int stage_result(const uint64_t* dev, uint32_t words) {
-  FDY_HIP(hipMemcpyAsync(g_stage.result(), dev, 8ull * words, hipMemcpyDeviceToHost, g_stage.lane.st));
-  FDY_HIP(hipStreamSynchronize(g_stage.lane.st));
+  FDY_HIP(hipMemcpyAsync(g_stage.result(), dev, 8ull * words, hipMemcpyDeviceToHost, g_stage.lane->st));
+  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
   return FDY_OK;
 }
 
@@ -297,7 +303,7 @@ int check_staged(const IndexArgs& ia, const uint64_t* lo, const uint64_t* hi, co
     return rc;
   }
   uint32_t blocks = 0;
-  hipError_t e = launch_table_check(ia, part.as<uint64_t>(), &blocks, g_stage.lane.st);
+  hipError_t e = launch_table_check(ia, part.as<uint64_t>(), &blocks, g_stage.lane->st);
   if (e == hipSuccess && stage_result(part.as<uint64_t>(), 2 * blocks) != FDY_OK) {
     *why = g_err;
     return FDY_E_HIP;
@@ -331,7 +337,7 @@ int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interv
   ia.shift = sh.shift;
   ia.block_sum = sums.as<uint64_t>();
   ia.total = sums.as<uint64_t>() + nblocks;
-  FDY_HIP(launch_index_count(ia, g_stage.lane.st));
+  FDY_HIP(launch_index_count(ia, g_stage.lane->st));
   rc = stage_result(ia.total, 1);
   if (rc) return rc;
   *total = *g_stage.result();
@@ -340,8 +346,8 @@ int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interv
   rc = dev_alloc(*out, *total * sizeof(RelocLine), "interval index lines");
   if (rc) return rc;
   ia.line = out->as<RelocLine>();
-  FDY_HIP(launch_index_place(ia, g_stage.lane.st));
-  FDY_HIP(hipStreamSynchronize(g_stage.lane.st));  // before the counts (and a caller's table) are freed
+  FDY_HIP(launch_index_place(ia, g_stage.lane->st));
+  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));  // before the counts (and a caller's table) are freed
   return FDY_OK;
 }
 
@@ -360,7 +366,7 @@ int place_roots(IndexArgs ia, const RootShape& sh, DevBuf* out, RelocDev* dev) {
   ia.block_sum = work.as<uint64_t>();
   ia.total = work.as<uint64_t>() + nblocks;
   ia.ends = reinterpret_cast<uint32_t*>(work.as<uint64_t>() + nblocks + 1);
-  FDY_HIP(launch_roots_count(ia, g_stage.lane.st));
+  FDY_HIP(launch_roots_count(ia, g_stage.lane->st));
   rc = stage_result(ia.total, 1);
   if (rc) return rc;
   const uint64_t total = *g_stage.result();
@@ -372,8 +378,8 @@ int place_roots(IndexArgs ia, const RootShape& sh, DevBuf* out, RelocDev* dev) {
   dev->line = ia.line = reinterpret_cast<RelocLine*>(out->as<uint8_t>() + root_bytes);
   dev->shift = sh.shift;
   dev->fence_shift = sh.fence_shift;
-  FDY_HIP(launch_roots_place(ia, g_stage.lane.st));
-  FDY_HIP(hipStreamSynchronize(g_stage.lane.st));  // before the counts (and a caller's table) are freed
+  FDY_HIP(launch_roots_place(ia, g_stage.lane->st));
+  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));  // before the counts (and a caller's table) are freed
   return FDY_OK;
 }
 
@@ -433,7 +439,7 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
     if (line_shape(span, n, root_lines_per_interval).nb > kMaxIndexLines)
       return err(FDY_E_INVALID, "interval index too large");
     if (n == 1) {  // one delta: no index
-      FDY_HIP(hipStreamSynchronize(g_stage.lane.st));
+      FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
     } else if (plan && n > kRootedIntervals) {
       uint64_t total = 0;
       rc = place_root_lines(ia, span, root_lines_per_interval, kMaxIndexLines, &out->index, &total, &d.shift);
