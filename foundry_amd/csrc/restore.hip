@@ -295,31 +295,24 @@ int stage_result(const uint64_t* dev, uint32_t words) {
 // check_table of the staged table at ia.lo (its arguments checked), by a
 // kernel.  A table at fault is walked on the host for its first fault.
 int check_staged(const IndexArgs& ia, const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo, uint32_t policy,
-                 uint64_t* off_bits, std::string* why) {
+                 uint64_t* off_bits) {
   DevBuf part;
   int rc = dev_alloc(part, 8 * kStageResults, "interval table check");
-  if (rc) {
-    *why = g_err;
-    return rc;
-  }
+  if (rc) return rc;
   uint32_t blocks = 0;
-  hipError_t e = launch_table_check(ia, part.as<uint64_t>(), &blocks, g_stage.lane->st);
-  if (e == hipSuccess && stage_result(part.as<uint64_t>(), 2 * blocks) != FDY_OK) {
-    *why = g_err;
-    return FDY_E_HIP;
-  }
-  if (e != hipSuccess) {
-    *why = std::string("the interval table's check failed: ") + hipGetErrorString(e);
-    return FDY_E_HIP;
-  }
+  FDY_HIP(launch_table_check(ia, part.as<uint64_t>(), &blocks, g_stage.lane->st));
+  rc = stage_result(part.as<uint64_t>(), 2 * blocks);
+  if (rc) return rc;
   uint64_t bad = 0;
   *off_bits = 0;
   for (uint32_t b = 0; b < blocks; ++b) {
     bad |= g_stage.result()[2 * b];
     *off_bits |= g_stage.result()[2 * b + 1];
   }
-  if (bad || ia.n > 0xFFFFFFF0ull || (hi[ia.n - 1] - lo[0]) >> 54) return check_table(lo, hi, nlo, ia.n, policy, off_bits, why);
-  return FDY_OK;
+  if (!bad && ia.n <= 0xFFFFFFF0ull && !((hi[ia.n - 1] - lo[0]) >> 54)) return FDY_OK;
+  std::string why;
+  rc = check_table(lo, hi, nlo, ia.n, policy, off_bits, &why);
+  return rc ? err(rc, why) : FDY_OK;
 }
 
 // The index of root lines of the table at ia.lo, ia.hi, ia.nlo (device
@@ -420,7 +413,13 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
     if (!rc) rc = stage_open();
     const uint64_t* const arrays[3] = {lo, hi, nlo};
     if (!rc) rc = stage_table(table.as<uint8_t>(), arrays, n);
-    if (rc) {
+    IndexArgs ia{};
+    ia.lo = table.as<uint64_t>();
+    ia.hi = ia.lo + n;
+    ia.nlo = ia.lo + 2 * n;
+    ia.n = n;
+    if (!rc && n > kHostCheck) rc = check_staged(ia, lo, hi, nlo, policy, &off_bits);
+    if (rc && rc != FDY_E_INVALID) {
       // No device for the table's check: the host's, so that a table at fault
       // is reported as such all the same.
       const std::string device_why = g_err;
@@ -428,13 +427,7 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
         if (const int bad = check_table(lo, hi, nlo, n, policy, &off_bits, &why)) return err(bad, why);
       return err(rc, device_why);
     }
-    IndexArgs ia{};
-    ia.lo = table.as<uint64_t>();
-    ia.hi = ia.lo + n;
-    ia.nlo = ia.lo + 2 * n;
-    ia.n = n;
-    if (n > kHostCheck) rc = check_staged(ia, lo, hi, nlo, policy, &off_bits, &why);
-    if (rc) return err(rc, why);
+    if (rc) return rc;
     const uint64_t span = hi[n - 1] - lo[0];
     if (line_shape(span, n, root_lines_per_interval).nb > kMaxIndexLines)
       return err(FDY_E_INVALID, "interval index too large");

@@ -10,6 +10,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from foundry_amd._lib import FoundryError
@@ -146,3 +147,17 @@ def test_restore_by_a_crowded_table(cuda, intervals):
         arch.restore()
         assert_restore_parity(arch, oracle.Restore(s.images(), table, policy=policy, threads=4))
         arch.close()
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="there is a device")
+def test_large_tables_at_fault_without_a_device():
+    """A table that the device would check (more than 32768 intervals) is
+    checked on the host where there is none: its fault is what is reported."""
+    n = 40000
+    lo = np.uint64(1 << 40) + np.uint64(4096) * np.arange(n, dtype=np.uint64)
+    hi = lo + np.uint64(4096)
+    hi[n // 2] = lo[n // 2]
+    with pytest.raises(FoundryError, match=f"interval {n // 2} is empty"):
+        RelocPlan(lo, hi, lo)
+    with pytest.raises(FoundryError, match="hipMalloc"):
+        RelocPlan(lo, lo + np.uint64(4096), lo)
