@@ -130,3 +130,43 @@ def test_empty_table_zero_words_and_refused_tables(cuda):
             RelocPlan(lo, hi, lo)
     with pytest.raises(FoundryError, match="policy"):
         RelocPlan(np.array([100], np.uint64), np.array([200], np.uint64), np.array([0], np.uint64), 2)
+
+
+@pytest.mark.parametrize("intervals", [0, 1, 2, 4096, 40000])
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 1, 5_000_003])
+def test_relocate_at_the_edge_of_small_calls(cuda, n, intervals):
+    """Calls of 1,048,576 words and fewer take one pair of words per thread,
+    larger ones four: both, both policies, 16-byte and 8-byte aligned arrays."""
+    print(f"[case] relocate words={n} intervals={intervals}", flush=True)
+    s = synth.SynthArchive(synth.preset(4, num_words=n, num_intervals=max(1, intervals), seed=0xC5 + intervals))
+    words = np.array(s.words(), copy=True)
+    lo, hi, nlo = (np.asarray(a)[:intervals] for a in s.intervals())
+    d_in = cuda.from_numpy(words.view(np.int64)).to("cuda")
+    for policy in (0, 1):
+        want = oracle.relocate_words(words, lo, hi, nlo, policy, threads=8)
+        plan = RelocPlan(lo, hi, nlo, policy)
+        for start in (0, 1):
+            d_out = cuda.full_like(d_in, -1)
+            plan.relocate(d_in.data_ptr() + 8 * start, d_out.data_ptr() + 8 * start, n - start)
+            cuda.cuda.synchronize()
+            np.testing.assert_array_equal(d_out.cpu().numpy().view(np.uint64)[start:], want[start:])
+        plan.close()
+
+
+@pytest.mark.parametrize("intervals", [1, 4096, 900_000])
+def test_relocate_in_place_over_several_chunks(cuda, intervals):
+    """In place on more words than one chunk per workgroup (8192 workgroups of
+    2048 words): a workgroup loads its next chunk before it has stored this one.
+    By one delta, the two-level index and the index of root lines."""
+    n = 8192 * 2048 + 2048 * 300 + 1
+    print(f"[case] relocate in place words={n} intervals={intervals}", flush=True)
+    s = synth.SynthArchive(synth.preset(4, num_words=n, num_intervals=intervals, seed=0xC6 + intervals))
+    words = np.array(s.words(), copy=True)
+    lo, hi, nlo = s.intervals()
+    plan = RelocPlan(lo, hi, nlo, 0)
+    d = cuda.from_numpy(words.view(np.int64)).to("cuda")
+    plan.relocate(d.data_ptr(), d.data_ptr(), n)
+    cuda.cuda.synchronize()
+    plan.close()
+    np.testing.assert_array_equal(d.cpu().numpy().view(np.uint64),
+                                  oracle.relocate_words(words, lo, hi, nlo, 0, threads=8))

@@ -11,6 +11,7 @@ import threading
 import numpy as np
 import pytest
 
+import graph_cases as GC
 from foundry_amd import synth
 from tests.parity import gpu_and_oracle
 
@@ -187,3 +188,43 @@ def test_short_sequences_with_tables(cuda, graphs, groups, nodes, blob):
             ref.switch(g)
         _same_live(arch, ref, [m[0] for m in own])
     arch.close()
+
+
+def test_sequences_in_the_serving_layout(cuda):
+    """A sequence that builds the tables, then a group graph on one group (the
+    archive packs its records and images, so the tables are another layout's),
+    sequences of the other groups and of all, and after the group graph another
+    restore and the first sequence again."""
+    from foundry_amd.graph import GroupGraph, Registry
+
+    print("[case] switch sequences before, in and after the serving layout", flush=True)
+    reg = Registry()
+    s = synth.SynthArchive(synth.preset(2, num_graphs=12, num_groups=3, nodes_per_graph=80, num_intervals=64,
+                                        diff_lo=0.1, diff_hi=0.1, sink_hash=reg.add_file(GC.PROBE_CO)))
+    arch, ref = gpu_and_oracle(s)
+    of = arch.groups()
+    templates = sorted(set(int(t) for t in of))
+    seq = [int(g) for g in synth.switch_sequence(5, 12, 60)]
+    others = [g for g in seq if of[g] != templates[0]]
+    assert len(others) >= 16
+
+    def run(targets, against):
+        arch.switch_sequence(targets)
+        for g in targets:
+            against.switch(g)
+        _same_live(arch, against, templates)
+
+    run(seq, ref)
+    gg = GroupGraph(arch, templates[0], reg, cuda.cuda.current_stream())
+    assert arch.info()["serving_layout"] == 1
+    ref.switch(templates[0])  # a new group graph is its template
+    run(others, ref)
+    run(seq, ref)  # the bound group's switches go through its group graph
+    run(others[::-1], ref)
+    gg.close()
+    arch.restore()
+    assert arch.info()["serving_layout"] == 0
+    _, again = gpu_and_oracle(s)
+    run(seq, again)
+    arch.close()
+    reg.close()

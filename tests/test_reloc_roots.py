@@ -2,8 +2,10 @@
 answer themselves, whose range holds one leaf (4 intervals), all seven (28) and one more (a tree of
 lines: 29, 60, 61, 900, 901), starts on the fences' unit and off it, one, two and
 256 entries more or less, a gap before every interval and none, both policies.
-On the CPU the host build and one lane's search, and on the GPU the device
-build and k_reloc's search by waves, against the oracle's binary search, bit for bit."""
+On the CPU the host build and one lane's search against the oracle's binary
+search, and on the GPU the device build against the host build, entry for entry
+and line for line, and k_reloc's searches by waves, through this index and
+through the index of root lines, against the oracle's, bit for bit."""
 import json
 import os
 import subprocess
@@ -14,9 +16,11 @@ import torch
 
 import oracle
 from foundry_amd._lib import FoundryError
-from foundry_amd.restore import RelocPlan
+from foundry_amd.restore import RelocPlan, relocate_words_static
 
-CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "_build", "reloc_roots_check")
+NATIVE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "_build")
+CHECK = os.path.join(NATIVE, "reloc_roots_check")
+BUILD_CHECK = os.path.join(NATIVE, "roots_build_check")
 
 
 def _run_of(rng, at, count, unit, gap):
@@ -92,6 +96,45 @@ def test_device_build_and_search(cuda, kind):
             cuda.cuda.synchronize()
             np.testing.assert_array_equal(d_out.cpu().numpy().view(np.uint64)[start:], want[start:])
         plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [k for k in KINDS if k != "one"])
+def test_search_through_root_lines(cuda, kind):
+    """k_reloc's search through an index of root lines (relocate_words_static)
+    over the same tables, the words shuffled so that the lookups of a wave end
+    in leaves, under one fence line and under several at once: in one small call
+    and in one of over a million words."""
+    rng = np.random.default_rng(KINDS.index(kind))
+    lo, hi, nlo, words = _table(kind, rng)
+    print(f"[case] root lines: {kind}, {len(lo)} intervals, {len(words)} words", flush=True)
+    words = rng.permutation(words)
+    for n in (len(words), (1 << 20) + 4097):
+        w = np.resize(words, n)
+        d_in = cuda.from_numpy(w.view(np.int64)).to("cuda")
+        for policy in (0, 1):
+            d_out = cuda.zeros_like(d_in)
+            relocate_words_static(lo, hi, nlo, d_in.data_ptr(), d_out.data_ptr(), n, policy)
+            cuda.cuda.synchronize()
+            np.testing.assert_array_equal(d_out.cpu().numpy().view(np.uint64),
+                                          oracle.relocate_words(w, lo, hi, nlo, policy, threads=8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+def test_device_build_equals_the_host_build(cuda, tmp_path, kind):
+    """Every root entry and line that the index kernels place is the host
+    build's (roots_build_check runs both)."""
+    lo, hi, nlo, _ = _table(kind, np.random.default_rng(KINDS.index(kind)))
+    print(f"[case] device build of the two-level index: {kind}, {len(lo)} intervals", flush=True)
+    t = str(tmp_path / "t.bin")
+    for policy in (0, 1):
+        np.concatenate([np.array([len(lo), policy], np.uint64), lo, hi, nlo]).tofile(t)
+        p = subprocess.run([BUILD_CHECK, t], capture_output=True, text=True, timeout=60)
+        assert p.returncode == 0, (p.returncode, p.stderr)
+        got = json.loads(p.stdout)
+        assert got["device_lines"] == got["lines"] and got["bad_roots"] == got["bad_lines"] == 0, got
+        assert kind not in ("crowded", "40000") or got["lines"] > 1000, got
 
 
 @pytest.mark.gpu
