@@ -91,16 +91,20 @@ struct UploadLane {
     st = nullptr;
     device = -1;
   }
-  bool open(int dev) {  // `dev` is the calling thread's device
-    if (device == dev) return true;
-    close();
-    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&ev[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) != hipSuccess) {
+  bool open(int dev, bool own_stream = true) {  // `dev` is the calling thread's device
+    if (device != dev) {
+      close();
+      if (hipEventCreateWithFlags(&ev[0], hipEventDisableTiming) != hipSuccess ||
+          hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) != hipSuccess) {
+        close();
+        return false;
+      }
+      device = dev;
+    }
+    if (own_stream && !st && hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
       close();
       return false;
     }
-    device = dev;
     return true;
   }
 };
@@ -227,7 +231,12 @@ int build_reloc_index(const uint64_t* lo, const uint64_t* hi, const uint64_t* nl
 // The upload of interval tables: pinned slots of their own (a program
 // that only builds plans need not hold the ring) and, per device, a lane that
 // the index kernels run on as well, so that nothing waits between the copy and
-// them.
+// them.  A process's first table goes without either: its arrays are copied
+// from where they lie, and the lane is the null stream (until a table comes
+// while work is queued there).  A stream takes 3 to 4 ms to create and the
+// slots 0.36 us per KB to touch first, where the one table of a process that
+// loads an archive takes 1.7 ms (10 intervals) to 2.7 (200,000) in all; with
+// both it took 5.0 to 7.2.
 // The lock holds from stage_open() until the index is built.  Tables of up to
 // 262,144 intervals fit three of the slots and are copied without a wait.
 constexpr uint64_t kStageSlot = 2ull << 20;
@@ -235,40 +244,65 @@ constexpr uint32_t kStageSlots = 4;
 constexpr uint32_t kStageResults = 2 * kTableBlocks;
 struct TableStage {
   std::mutex mu;
-  uint8_t* host = nullptr;  // the slots, then kStageResults words for results
+  bool opened = false;      // by an earlier table
+  uint8_t* host = nullptr;  // the slots, then kStageResults words for results; null where none can be pinned
+  uint64_t local[kStageResults];  // results where there are no slots
   std::map<int, UploadLane> lanes;
   UploadLane* lane = nullptr;  // the open stage's, or the last one's
-  uint64_t* result() const { return reinterpret_cast<uint64_t*>(host + kStageSlots * kStageSlot); }
+  bool in_flight = false;      // copies or kernels of the lane's not yet waited for
+  uint64_t* result() { return host ? reinterpret_cast<uint64_t*>(host + kStageSlots * kStageSlot) : local; }
 };
 TableStage g_stage;
 
-int stage_open() {
-  if (!g_stage.host) {
-    void* p = nullptr;
-    const size_t bytes = kStageSlots * kStageSlot + 8 * kStageResults;
-    if (hipHostMalloc(&p, bytes, hipHostMallocPortable) != hipSuccess) {
-      (void)hipGetLastError();
-      p = std::malloc(bytes);  // unpinned: copies that the runtime stages
-      if (!p) return err(FDY_E_NOMEM, "interval table staging of " + std::to_string(bytes) + " bytes");
-    }
-    g_stage.host = static_cast<uint8_t*>(p);
-  }
-  int dev = 0;
-  FDY_HIP(hipGetDevice(&dev));
-  UploadLane& lane = g_stage.lanes[dev];
-  if (!lane.open(dev)) {
-    (void)hipGetLastError();
-    return err(FDY_E_HIP, "cannot create an upload stream or event");
-  }
-  // A call that failed part-way may have left copies out of the slots.
-  if (g_stage.lane) FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
-  g_stage.lane = &lane;
+// Waits for what the lane has been given.
+int stage_wait() {
+  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
+  g_stage.in_flight = false;
   return FDY_OK;
 }
 
-// The three arrays of n words to `dst`, end to end, in stream order.
+int stage_open() {
+  if (g_stage.opened && !g_stage.host) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kStageSlots * kStageSlot + 8 * kStageResults, hipHostMallocPortable) == hipSuccess)
+      g_stage.host = static_cast<uint8_t*>(p);
+    else
+      (void)hipGetLastError();
+  }
+  g_stage.opened = true;
+  int dev = 0;
+  FDY_HIP(hipGetDevice(&dev));
+  // A call that failed part-way may have left copies out of the slots.
+  if (g_stage.in_flight) {
+    FDY_HIP(hipSetDevice(g_stage.lane->device));
+    const int rc = stage_wait();
+    FDY_HIP(hipSetDevice(dev));
+    if (rc) return rc;
+  }
+  UploadLane& lane = g_stage.lanes[dev];
+  const bool idle = !lane.st && hipStreamQuery(nullptr) == hipSuccess;
+  if (!lane.st && !idle) (void)hipGetLastError();  // not ready
+  if (!lane.open(dev, !idle)) {
+    (void)hipGetLastError();
+    return err(FDY_E_HIP, "cannot create an upload stream or event");
+  }
+  g_stage.lane = &lane;
+  g_stage.in_flight = true;
+  return FDY_OK;
+}
+
+// The three arrays of n words to `dst`, end to end, in stream order; the arrays
+// are free again on return.
 int stage_table(uint8_t* dst, const uint64_t* const src[3], uint64_t n) {
   const hipStream_t st = g_stage.lane->st;
+  if (!g_stage.host) {
+    hipError_t e = hipSuccess;
+    for (uint32_t a = 0; a < 3 && e == hipSuccess; ++a)
+      e = hipMemcpyAsync(dst + 8 * n * a, src[a], 8 * n, hipMemcpyHostToDevice, st);
+    const int rc = stage_wait();
+    FDY_HIP(e);
+    return rc;
+  }
   uint32_t k = 0;
   for (uint32_t a = 0; a < 3; ++a)
     for (uint64_t at = 0; at < 8 * n; at += kStageSlot, ++k) {
@@ -288,8 +322,7 @@ int stage_table(uint8_t* dst, const uint64_t* const src[3], uint64_t n) {
 // device, at g_stage.result() once the kernels have run.
 int stage_result(const uint64_t* dev, uint32_t words) {
   FDY_HIP(hipMemcpyAsync(g_stage.result(), dev, 8ull * words, hipMemcpyDeviceToHost, g_stage.lane->st));
-  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
-  return FDY_OK;
+  return stage_wait();
 }
 
 // check_table of the staged table at ia.lo (its arguments checked), by a
@@ -340,8 +373,7 @@ int place_root_lines(IndexArgs ia, uint64_t span, uint64_t root_lines_per_interv
   if (rc) return rc;
   ia.line = out->as<RelocLine>();
   FDY_HIP(launch_index_place(ia, g_stage.lane->st));
-  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));  // before the counts (and a caller's table) are freed
-  return FDY_OK;
+  return stage_wait();  // before the counts (and a caller's table) are freed
 }
 
 // A table's two-level index on the device: its lines counted, placed and
@@ -372,8 +404,7 @@ int place_roots(IndexArgs ia, const RootShape& sh, DevBuf* out, RelocDev* dev) {
   dev->shift = sh.shift;
   dev->fence_shift = sh.fence_shift;
   FDY_HIP(launch_roots_place(ia, g_stage.lane->st));
-  FDY_HIP(hipStreamSynchronize(g_stage.lane->st));  // before the counts (and a caller's table) are freed
-  return FDY_OK;
+  return stage_wait();  // before the counts (and a caller's table) are freed
 }
 
 // Plans of more intervals keep an index of root lines.  Their root entries
@@ -432,7 +463,7 @@ int build_reloc_plan(const uint64_t* lo, const uint64_t* hi, const uint64_t* nlo
     if (line_shape(span, n, root_lines_per_interval).nb > kMaxIndexLines)
       return err(FDY_E_INVALID, "interval index too large");
     if (n == 1) {  // one delta: no index
-      FDY_HIP(hipStreamSynchronize(g_stage.lane->st));
+      rc = stage_wait();
     } else if (plan && n > kRootedIntervals) {
       uint64_t total = 0;
       rc = place_root_lines(ia, span, root_lines_per_interval, kMaxIndexLines, &out->index, &total, &d.shift);

@@ -9,6 +9,7 @@ through the index of root lines, against the oracle's, bit for bit."""
 import json
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -204,3 +205,41 @@ def test_large_tables_at_fault_without_a_device():
         RelocPlan(lo, hi, lo)
     with pytest.raises(FoundryError, match="hipMalloc"):
         RelocPlan(lo, lo + np.uint64(4096), lo)
+
+
+_FIRST_TABLES = """
+import numpy as np, torch
+import oracle
+from foundry_amd.restore import RelocPlan
+rng = np.random.default_rng(9)
+d = None
+for k, (n, busy) in enumerate([(300_000, False), (300_000, False), (40_000, True), (300_000, False), (10, True)]):
+    size = rng.integers(1, 64, n).astype(np.uint64) * np.uint64(256)
+    hi = np.uint64(1 << 44) + np.cumsum(size, dtype=np.uint64)
+    lo = hi - size
+    nlo = rng.permutation(n).astype(np.uint64) << np.uint64(20)
+    words = np.concatenate([lo, hi, hi - np.uint64(1)])
+    d_in = torch.from_numpy(words.view(np.int64)).cuda()
+    d_out = torch.zeros_like(d_in)
+    torch.cuda.synchronize()
+    if busy:
+        torch.cuda._sleep(50_000_000)
+    plan = RelocPlan(lo, hi, nlo)
+    plan.relocate(d_in.data_ptr(), d_out.data_ptr(), len(words))
+    torch.cuda.synchronize()
+    assert np.array_equal(d_out.cpu().numpy().view(np.uint64), oracle.relocate_words(words, lo, hi, nlo, 0)), (k, n)
+    plan.close()
+    print("table", k, n, "same", flush=True)
+"""
+
+
+@pytest.mark.gpu
+def test_first_tables_of_a_process():
+    """A process's first table is copied from where it lies, later ones go
+    through the staging slots (several rounds of them here), on the null stream
+    or, with work queued there, on the stage's own: each relocates as the
+    oracle does."""
+    print("[case] the first tables of a process", flush=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    p = subprocess.run([sys.executable, "-c", _FIRST_TABLES], cwd=root, capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0 and p.stdout.count("same") == 5, (p.returncode, p.stdout, p.stderr)
