@@ -561,16 +561,21 @@ __device__ __forceinline__ uint64_t name_crc(const Strings& S, const E& e, const
 template <class E>
 __device__ __forceinline__ void node_pointers(const E& e, const RelocDev& r, uint64_t* p0, uint64_t* p1) {
   const uint8_t type = e.type();
-  *p0 = 0;
-  *p1 = 0;
+  uint64_t w[2] = {0, 0};
+  uint32_t m = 0;  // the words to relocate
   if (type == FDY_NODE_MEMSET) {
-    *p0 = reloc_word(r, e.u64(FDY_MSOFF_DST));
+    w[0] = e.u64(FDY_MSOFF_DST);
+    m = 1;
   } else if (type == FDY_NODE_MEMCPY) {
-    const uint64_t dst = e.u64(FDY_MCOFF_DST), src = e.u64(FDY_MCOFF_SRC);
     const int32_t dt = (int32_t)e.u32(FDY_MCOFF_DST_MEMTYPE), st = (int32_t)e.u32(FDY_MCOFF_SRC_MEMTYPE);
-    *p0 = (dt == FDY_MEMTYPE_DEVICE || dt == FDY_MEMTYPE_UNIFIED) ? reloc_word(r, dst) : dst;
-    *p1 = (st == FDY_MEMTYPE_DEVICE || st == FDY_MEMTYPE_UNIFIED) ? reloc_word(r, src) : src;
+    w[0] = e.u64(FDY_MCOFF_DST);
+    w[1] = e.u64(FDY_MCOFF_SRC);
+    m = (dt == FDY_MEMTYPE_DEVICE || dt == FDY_MEMTYPE_UNIFIED ? 1u : 0u) |
+        (st == FDY_MEMTYPE_DEVICE || st == FDY_MEMTYPE_UNIFIED ? 2u : 0u);
   }
+  if (m) reloc_pair(r, w, m);
+  *p0 = w[0];
+  *p1 = w[1];
 }
 
 template <class EA, class EB>

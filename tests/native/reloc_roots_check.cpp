@@ -8,7 +8,8 @@
 // WORDS: u64 words.  OUT: the relocated words; then one JSON line on stdout
 // with the index's shape: root entries, whether their fences are exact,
 // lines, and the entries by what is below them ("direct": nothing, "flat":
-// leaves alone, "deep": a tree).
+// leaves alone, "deep": a tree), and the words of pairs that reloc_pair moves
+// otherwise than reloc_word.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -58,19 +59,28 @@ int main(int argc, char** argv) {
   }
   std::vector<uint64_t> out(w.size());
   for (size_t i = 0; i < w.size(); ++i) out[i] = reloc_word(d, w[i]);
+  // Two words at once, either or both of them: each as by itself.
+  uint64_t bad_pairs = 0;
+  for (size_t i = 0; i < w.size(); ++i)
+    for (uint32_t mask = 0; mask < 4; ++mask) {
+      const size_t j = (i * 7 + 3) % w.size();
+      uint64_t p[2] = {w[i], w[j]};
+      reloc_pair(d, p, mask);
+      bad_pairs += p[0] != (mask & 1 ? out[i] : w[i]) || p[1] != (mask & 2 ? out[j] : w[j]);
+    }
   FILE* f = std::fopen(argv[3], "wb");
   if (!f || std::fwrite(out.data(), 8, out.size(), f) != out.size()) {
     std::perror(argv[3]);
     return 2;
   }
   std::fclose(f);
-  std::printf("{\"roots\": %zu, \"exact\": %d, \"lines\": %zu, \"direct\": %llu, \"flat\": %llu, \"deep\": %llu}\n", x.root.size(),
+  std::printf("{\"roots\": %zu, \"exact\": %d, \"lines\": %zu, \"direct\": %llu, \"flat\": %llu, \"deep\": %llu, \"bad_pairs\": %llu}\n", x.root.size(),
               (int)(n == 0 || root_shape(lo, hi, n, [&] {
                       uint64_t bits = 0;
                       for (uint64_t i = 0; i < n; ++i) bits |= lo[i] - lo[0];
                       return bits;
                     }()).exact),
               x.line.size(), (unsigned long long)direct, (unsigned long long)(x.root.size() - direct - deep),
-              (unsigned long long)deep);
+              (unsigned long long)deep, (unsigned long long)bad_pairs);
   return 0;
 }

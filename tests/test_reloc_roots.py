@@ -78,6 +78,7 @@ def test_host_build_and_search(tmp_path, kind):
         assert kind not in ("aligned", "1021", "40000") or (shape["exact"] and shape["flat"] > 0), shape
         assert kind != "bytes" or not shape["exact"], shape
         assert kind == "one" or shape["direct"] > 0, shape
+        assert shape["bad_pairs"] == 0, shape
         assert kind not in ("aligned", "unaligned", "bytes", "crowded") or shape["deep"] > 0, shape
         np.testing.assert_array_equal(np.fromfile(o, np.uint64), oracle.relocate_words(words, lo, hi, nlo, policy))
 
