@@ -1738,7 +1738,7 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
 //   Bound by requests: 4 ps each over the GPU where they hit the L2s, 18 ps
 // where they miss them, whatever their size up to 128 B (250 and 55 G/s
 // measured over 4 MB and 200 MB).  So the index is small (25 to 53 bytes per
-// interval) and one more, cached, read deep.  20.5 M
+// interval of the workloads' tables), and a lookup two reads that hit the L2s.  20.5 M
 // words with 25% pointers by 40,000 intervals: 97 us, where 16 root lines of
 // 64 B per interval (41 MB) read by one lane each took 136 us; eight lanes per
 // 128-byte line were slower than four per 64 bytes (an L2 hit delivers 10.5
@@ -3006,6 +3006,13 @@ __global__ __launch_bounds__(kFillThreads) void k_fill(FillArgs a) {
 // A wave's words lie in LDS meanwhile, with a list of those inside the
 // table's range (the pointers: 40% on the relocation-heavy workload), which
 // are searched there.
+//   The output is stored past the caches.  Words in no cache (164 MB, 8 inputs
+// and outputs in turn) by one interval: 56.4 us, with cached stores 4 M words
+// 13.3 -> 15.0 us and 16 M 43.5 -> 46.7.  Its reader finds nothing in the caches
+// for it: a relocation and a copy of its output take the same either way up to
+// 500,000 words (7.8 to 8.0 us), 8.9 against 8.3 at a million, 96.5 against 109
+// at 16 M in turn, but 91.5 against 79 where one 128 MB output comes again and
+// again and just fits the MALL.
 constexpr uint32_t kRelocLines = 8;   // lines in flight per quad
 
 template <bool kRooted, uint32_t kPairs>

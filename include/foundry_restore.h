@@ -275,10 +275,14 @@ int fdy_get_live(fdy_archive* a, void* stream, uint32_t template_graph, uint64_t
 /* Standalone relocation of packed u64 words already in device memory
  * (in and out may alias).  The plan holds the table's interval search
  * structure: up to 786,432 intervals, root entries of 16 B over lines of 64 B
- * and the table itself (50 to 80 B per interval in all); past that, about 16
- * root lines of 64 B per interval (2M intervals: about 2 GB of device
- * memory).  The table is checked on the host and the index built on the
- * current device (only the table is uploaded); returns when it is built. */
+ * and the table itself (24 B per interval): 64 to 77 B per interval in all for
+ * 40,000 allocations of mixed sizes, 49 for 200,000, at most about 150; a few
+ * intervals may take up to 512 KB (32,768 entries, which make their places
+ * exact) or an entry per 2^31 bytes of span.  Past that, about 16 root lines
+ * of 64 B per interval (2M intervals: about 2 GB of device memory).  The table
+ * is checked on the host (past 32,768 intervals on the device, with the same
+ * refusals) and the index built on the current device (only the table is
+ * uploaded); returns when it is built. */
 int fdy_reloc_plan_create(const uint64_t* lo, const uint64_t* hi, const uint64_t* new_lo, uint64_t n,
                           uint32_t policy, fdy_reloc_plan** out);
 int fdy_reloc_plan_destroy(fdy_reloc_plan* p);

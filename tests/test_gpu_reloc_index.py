@@ -1,14 +1,15 @@
-"""The interval index built on the device (fdy_reloc_plan_create: the
-builder of foundry_amd/csrc/reloc_index.h run as kernels, one thread per
-root line) against the host build of the same table
+"""A plan's table as an index of root lines, built on the device
+(fdy_reloc_plan_lines: the builder of foundry_amd/csrc/reloc_index.h run as
+kernels, one thread per root line; past 786,432 intervals it is the index that
+the plan searches) against the host build of the same table
 (tests/native/reloc_index_check, the same builder on the CPU, which the CPU
 tests pin against the oracle's search): equal line for line, 16 root lines
-per interval as in every plan, on tables shaped to reach every kind of line:
+per interval as in every large plan, on tables shaped to reach every kind of line:
 fence lines several levels deep (dense tiny intervals beside a huge one),
 random gaps with abutting intervals, the widest root lines over a sparse
 span, one interval, a table at the top of the address space, and the
 relocation-heavy workload's interval mix.  Each plan then relocates its
-table's edge words as the oracle does."""
+table's edge words, through the index it searches, as the oracle does."""
 import ctypes as C
 import os
 import subprocess

@@ -1,6 +1,7 @@
-"""The interval index (foundry_amd/csrc/reloc_index.h) and its search
-(reloc_batch in foundry_amd/csrc/restore_dev.h, the code the kernels run),
-executed on the CPU by tests/native/reloc_index_check and compared with the
+"""The index of root lines (foundry_amd/csrc/reloc_index.h) and its search by
+one lane (reloc_batch in foundry_amd/csrc/restore_dev.h; on the GPU a call's odd
+last word takes it, the others k_reloc's search by waves, which
+test_reloc_roots.py holds to the oracle), executed on the CPU by tests/native/reloc_index_check and compared with the
 oracle's binary search (oracle.cpp relocate_word, which follows the
 reference's relocation rule) on tables shaped to reach every kind of line:
 leaves, fence lines one and several levels deep, lines wider than any
