@@ -659,6 +659,7 @@ uint64_t seq_layout(fdy_archive* a) {
 // results are settled).
 int fill_live(fdy_archive* a, hipStream_t s) {
   const uint32_t G = a->G;
+  FDY_HIP(hipSetDevice(a->device));
   std::vector<uint64_t> lbase(G, 0);
   uint64_t live_words = 0;
   for (uint32_t g = 0; g < G; ++g)
@@ -1533,9 +1534,8 @@ int fdy_switch_sequence(fdy_archive* a, const uint32_t* targets, uint64_t n, voi
     if (a->seq_ready) {
       tiles = follow_seq_tables(a, s);
     } else if (n >= kSeqSwitches && !capturing(s)) {
-      rc = build_seq_tables(a, s);
-      if (rc) return rc;
-      tiles = true;
+      tiles = build_seq_tables(a, s) == FDY_OK;  // else by layers, which need none
+      if (!tiles) (void)hipGetLastError();
     }
   }
   if (tiles) {
