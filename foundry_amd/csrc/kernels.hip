@@ -3006,13 +3006,12 @@ __global__ __launch_bounds__(kFillThreads) void k_fill(FillArgs a) {
 // A wave's words lie in LDS meanwhile, with a list of those inside the
 // table's range (the pointers: 40% on the relocation-heavy workload), which
 // are searched there.
-//   The output is stored past the caches.  Words in no cache (164 MB, 8 inputs
-// and outputs in turn) by one interval: 56.4 us, with cached stores 4 M words
-// 13.3 -> 15.0 us and 16 M 43.5 -> 46.7.  Its reader finds nothing in the caches
-// for it: a relocation and a copy of its output take the same either way up to
-// 500,000 words (7.8 to 8.0 us), 8.9 against 8.3 at a million, 96.5 against 109
-// at 16 M in turn, but 91.5 against 79 where one 128 MB output comes again and
-// again and just fits the MALL.
+//   The output is stored past the caches: by one interval, several buffers in
+// turn, 4 M words take 13.3 us (cached stores 15.0), 16 M 43.5 (46.7).  Its
+// reader then finds none of it in the caches: a relocation and a copy of its
+// output take 7.8 to 8.0 us either way up to 500,000 words, 8.9 (8.3) at a
+// million and 96.5 (109) at 16 M in turn, but 91.5 (79) where one 128 MB output
+// is written over and over and just fits the MALL.
 constexpr uint32_t kRelocLines = 8;   // lines in flight per quad
 
 template <bool kRooted, uint32_t kPairs>
